@@ -1,0 +1,520 @@
+"""Workloads over which the speed of the attention path is measured.
+
+Each case is one call, or one short chain of calls, that a denoising step of a
+Wan-shaped video DiT makes: dense attention, block-sparse attention with the
+spatial token reorder around it, the sampled and the exact route estimate, the
+matrix-sparse backend's step and bootstrap with their tile statistics, and a
+forward of the DiT itself.  Token counts come from latent grids
+(frames x height x width); Q and K are 0.5 N(0,1) noise around a centroid
+shared by the tokens of a block or tile, V is N(0,1).
+"""
+
+from __future__ import annotations
+
+import math
+
+import torch
+import torch.nn.functional as F
+
+from dit_sparse_atten_amd import ops
+from dit_sparse_atten_amd.attention_backends import DenseBackend
+from dit_sparse_atten_amd.attention_backends.spatial import build_spatial_layout
+from dit_sparse_atten_amd.wan_dit import WanDiT, WanDiTConfig, rope_cos_sin
+
+HEAD_DIM = 128
+BLOCK = 128
+SAMPLES = 16
+DTYPES = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
+TEXT_TOKENS = 512
+MAX_FLOPS = 4.5e13       # of any case, the largest listed one's
+MAX_FLOPS_FP32 = 2.0e12  # fp32 runs at a sixteenth of the 16-bit rate
+
+
+# ---------------------------------------------------------------------------
+# Cases
+# ---------------------------------------------------------------------------
+
+def _case(kind, grid, heads, dtype="bf16", **more):
+    frames, height, width = grid
+    return {"kind": kind, "frames": frames, "height": height, "width": width, "heads": heads,
+            "dtype": dtype, **more}
+
+
+def listed():
+    return [
+        # The CPU reference configuration, whole: 1,024 tokens, 8 x 8 tiles,
+        # float32.  Launches and latency.
+        _case("tile", (4, 16, 16), 12, "fp32", tile_h=8, tile_w=8, name="tile_1k_fp32"),
+        # A single latent image of 3,600 tokens in 40 heads (720p, one frame):
+        # the sparse call and its route update at the short end.
+        _case("sparse", (1, 45, 80), 40, reorder=False, name="sparse_3k6"),
+        _case("update", (1, 45, 80), 40, previous=False, name="update_3k6"),
+        # The classifier-free-guidance pair of Wan2.1-1.3B at 480p, 81 frames:
+        # layer 0 and every route above the dense threshold.
+        _case("dense", (21, 30, 52), 12, batch=2, name="dense_480p_cfg"),
+        # Float32 through the dense backend, as parity checks of a model run it.
+        _case("dense", (4, 30, 30), 12, "fp32", batch=1, name="dense_3k6_fp32"),
+        # Wan2.1-14B at 720p, 61 frames: the sparse call between route updates.
+        _case("sparse", (16, 45, 80), 40, reorder=False, name="sparse_720p"),
+        # Wan2.1-1.3B at 480p in float16, with the Morton reorder and restore
+        # around the sparse call; 32,760 tokens leave a partial last block.
+        _case("sparse", (21, 30, 52), 12, "fp16", reorder=True, name="sparse_480p_reorder"),
+        # The sampled route update every second step, from a previous route.
+        _case("update", (16, 45, 80), 40, previous=True, name="update_720p"),
+        # The default (exact) bootstrap: dense attention, block mass, route.
+        _case("exact", (21, 30, 52), 12, name="exact_480p"),
+        # The matrix-sparse backend's step at 720p (9 x 8 tiles): attention on
+        # the kept tiles, its statistics, the next route.
+        _case("tile", (16, 45, 80), 40, tile_h=9, tile_w=8, name="tile_720p"),
+        # Its dense bootstrap with 6 x 10 tiles, 14,400 tokens.
+        _case("boot", (4, 60, 60), 40, tile_h=6, tile_w=10, name="boot_14k"),
+        # Two blocks of the 1.3B DiT with embeddings and head at 480p.
+        _case("dit", (21, 30, 52), 12, layers=2, name="dit_480p"),
+    ]
+
+
+def draw(rng):
+    """One more case: any kind, 512 to 57,600 tokens (log-uniform), 3 to 40
+    heads, odd grids included."""
+    kind = rng.choice(("dense", "sparse", "sparse", "update", "exact", "tile", "tile", "boot",
+                       "dit"))
+    dtype = rng.choice(("bf16", "bf16", "fp16"))
+    more = {}
+    if kind in ("tile", "boot"):
+        # Tiles as the backend's 64-token target picks them: near square,
+        # 48 to 104 tokens.
+        while True:
+            tile_h, tile_w = rng.randint(5, 13), rng.randint(5, 13)
+            if 48 <= tile_h * tile_w <= 104:
+                break
+        more = {"tile_h": tile_h, "tile_w": tile_w}
+        steps = (tile_h, tile_w)
+    else:
+        steps = (1, 1)
+    if kind in ("dense", "tile") and rng.random() < 0.25:
+        dtype = "fp32"
+    if kind == "dense":
+        more["batch"] = rng.choice((1, 2))
+    elif kind == "sparse":
+        more["reorder"] = rng.random() < 0.5
+    elif kind == "update":
+        more["previous"] = rng.random() < 0.5
+    elif kind == "dit":
+        more["layers"] = rng.choice((1, 2))
+        dtype = "bf16"
+    target = math.exp(rng.uniform(math.log(512), math.log(57600)))
+    height = steps[0] * max(1, round(rng.uniform(12, 48) / steps[0]))
+    width = steps[1] * max(1, round(rng.uniform(12, 80) / steps[1]))
+    while height * width > target and height > steps[0]:
+        height -= steps[0]
+    while height * width > target and width > steps[1]:
+        width -= steps[1]
+    frames = max(1, min(21, round(target / (height * width))))
+    heads = 12 if kind == "dit" else rng.choice((3, 5, 12, 24, 40))
+    case = _case(kind, (frames, height, width), heads, dtype, **more)
+    limit = MAX_FLOPS_FP32 if dtype == "fp32" else MAX_FLOPS
+    while work(case)["flops"] > limit:
+        if case["heads"] > 3 and kind != "dit":
+            case["heads"] = max(3, case["heads"] // 2)
+        elif case["frames"] > 1:
+            case["frames"] -= 1
+        else:
+            case["height"] -= steps[0]
+    return case
+
+
+def _shape(case):
+    tokens = case["frames"] * case["height"] * case["width"]
+    return tokens, case["heads"], DTYPES[case["dtype"]]
+
+
+def _frame_tokens(case):
+    return case["height"] * case["width"]
+
+
+# ---------------------------------------------------------------------------
+# Inputs
+# ---------------------------------------------------------------------------
+
+def _generator(seed):
+    return torch.Generator(device="cuda").manual_seed(int(seed))
+
+
+def _qkv(case, group, generator):
+    """Q, K, V [B, T, H, D] as views of head-major storage, the layout Wan's
+    attention processor hands over; one centroid per `group` tokens."""
+    tokens, heads, dtype = _shape(case)
+    batch = case.get("batch", 1)
+    groups = -(-tokens // group)
+    ids = torch.arange(tokens, device="cuda") // group
+
+    def clustered():
+        x = torch.randn((batch, heads, tokens, HEAD_DIM), device="cuda", generator=generator)
+        c = torch.randn((batch, heads, groups, HEAD_DIM), device="cuda", generator=generator)
+        return x.mul_(0.5).add_(c[:, :, ids]).to(dtype).transpose(1, 2)
+
+    q, k = clustered(), clustered()
+    v = torch.randn((batch, heads, tokens, HEAD_DIM), device="cuda", generator=generator)
+    return q, k, v.to(dtype).transpose(1, 2)
+
+
+def _rope_qkv(case, generator):
+    """N(0,1) Q/K/V with the 3D rotary embedding on Q and K."""
+    tokens, heads, dtype = _shape(case)
+    shape = (case["batch"], heads, tokens, HEAD_DIM)
+    table = rope_cos_sin((case["frames"], case["height"], case["width"]), HEAD_DIM, device="cuda")
+    cos, sin = table[..., 0], table[..., 1]
+
+    def rotated():
+        x = torch.randn(shape, device="cuda", generator=generator)
+        a, b = x[..., 0::2], x[..., 1::2]
+        return torch.stack((a * cos - b * sin, a * sin + b * cos), dim=-1).reshape(shape)
+
+    q, k = rotated(), rotated()
+    v = torch.randn(shape, device="cuda", generator=generator)
+    return tuple(x.to(dtype).transpose(1, 2) for x in (q, k, v))
+
+
+def _random_route(heads, blocks, sink, generator):
+    """Bernoulli(0.625) key blocks per row, the diagonal and the first-frame
+    sink always kept."""
+    route = torch.rand((heads, blocks, blocks), device="cuda", generator=generator) < 0.625
+    route |= torch.eye(blocks, dtype=torch.bool, device="cuda")
+    route[:, :, :sink] = True
+    return route
+
+
+def _tile_counts(case):
+    tile = case["tile_h"] * case["tile_w"]
+    return tile, _shape(case)[0] // tile, _frame_tokens(case) // tile
+
+
+def _model_inputs(case, generator):
+    """(config, latents, embedded-text input) of the DiT case."""
+    config = WanDiTConfig(layers=case["layers"])
+    latents = torch.randn((1, config.in_channels, case["frames"], 2 * case["height"],
+                           2 * case["width"]), device="cuda", generator=generator)
+    text = torch.randn((1, TEXT_TOKENS, config.text_dim), device="cuda", generator=generator)
+    return config, latents.to(torch.bfloat16), text.to(torch.bfloat16)
+
+
+def prepare(case, seed):
+    generator = _generator(seed)
+    tokens, heads, _ = _shape(case)
+    kind = case["kind"]
+    state = {"case": case}
+    if kind == "dit":
+        config, latents, text = _model_inputs(case, generator)
+        model = WanDiT(config, device="cuda", seed=seed)
+        return {**state, "model": model, "latents": latents, "context": model.embed_text(text),
+                "backend": DenseBackend()}
+    if kind == "dense":
+        q, k, v = _rope_qkv(case, generator)
+        return {**state, "q": q, "k": k, "v": v, "backend": DenseBackend()}
+    if kind in ("tile", "boot"):
+        tile, tiles, sink = _tile_counts(case)
+        # Tile-major tokens, as the backend's reorder leaves them.
+        q, k, v = (x.contiguous() for x in _qkv(case, tile, generator))
+        state.update(q=q, k=k, v=v, sink=sink)
+        if kind == "tile":
+            state["route"] = _random_route(heads, tiles, sink, generator)
+        return state
+    q, k, v = _qkv(case, BLOCK, generator)
+    state.update(q=q, k=k, v=v, sink=-(-_frame_tokens(case) // BLOCK))
+    blocks = -(-tokens // BLOCK)
+    if kind == "sparse":
+        state["csr"] = ops.route_to_csr(_random_route(heads, blocks, state["sink"], generator))
+        if case["reorder"]:
+            layout = build_spatial_layout((case["frames"], case["height"], case["width"]), BLOCK,
+                                          16)
+            layout.neighbors(q.device)  # puts the layout's tables on the device
+            state["layout"] = layout
+    elif kind == "update" and case["previous"]:
+        state["previous"] = _random_route(heads, blocks, state["sink"], generator)
+    return state
+
+
+# ---------------------------------------------------------------------------
+# One pass
+# ---------------------------------------------------------------------------
+
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "dit":
+        return state["model"](state["latents"], 882.0, state["context"], state["backend"])
+    q, k, v = state["q"], state["k"], state["v"]
+    if kind == "dense":
+        return state["backend"](q, k, v, dtype=q.dtype)
+    if kind == "sparse":
+        layout = state.get("layout")
+        if layout is None:
+            return ops.bsa_fwd(q, k, v, state["csr"])
+        q, k, v = layout.reorder_qkv(q, k, v)
+        return layout.restore(ops.bsa_fwd(q, k, v, state["csr"]))
+    if kind == "update":
+        mass = ops.sampled_block_mass(q, k, BLOCK, SAMPLES)
+        route, counts = ops.route_select(mass, 0.95, 0.625, previous=state.get("previous"),
+                                         persistence=0.5, sink_blocks=state["sink"])
+        # The CSR's column list is the route's cells in order, valid up to the
+        # device-side total only, so the route stands for it in the results.
+        csr = ops.route_to_csr(route, counts)
+        return {"mass": mass, "route": route, "counts": counts, "row_ptr": csr.row_ptr}
+    if kind == "exact":
+        out, lse, mass = ops.bsa_fwd_block_mass(q, k, v)
+        route, counts = ops.route_select(mass, 0.90, 0.625, sink_blocks=state["sink"])
+        csr = ops.route_to_csr(route, counts)
+        return {"out": out, "lse": lse, "mass": mass, "route": route, "counts": counts,
+                "row_ptr": csr.row_ptr}
+    tile_shape = (case["tile_h"], case["tile_w"])
+    if kind == "boot":
+        out, lse, stats = ops.bsa_fwd_tile_stats(q, k, v, None, tile_shape)
+        route, counts = ops.route_select(stats["mass"], 0.90, 0.625, sink_blocks=state["sink"])
+    else:
+        csr = ops.route_to_csr(state["route"], block_size=tile_shape[0] * tile_shape[1])
+        out, lse, stats = ops.bsa_fwd_tile_stats(q, k, v, csr, tile_shape)
+        route, counts = ops.drop_low_mass(state["route"], stats["mass"], 0.1, state["sink"])
+    return {"out": out, "lse": lse, "route": route, "counts": counts, **stats}
+
+
+# ---------------------------------------------------------------------------
+# What a pass cannot do without, and how far two correct ones may differ
+# ---------------------------------------------------------------------------
+
+def _kept(units, sink):
+    """Expected kept share of a Bernoulli route with its diagonal and sink."""
+    free = max(0, units - sink)
+    return (sink + free * (0.625 + 0.375 / units)) / units
+
+
+def work(case):
+    tokens, heads, dtype = _shape(case)
+    size = torch.empty((), dtype=dtype).element_size()
+    kind = case["kind"]
+    rows = case.get("batch", 1) * heads * tokens
+    tensor = rows * HEAD_DIM * size
+    pairs = 4.0 * HEAD_DIM * rows * tokens  # flops of dense attention
+    blocks = -(-tokens // BLOCK)
+    cells = heads * blocks * blocks
+    if kind == "dense":
+        return {"bytes": 4 * tensor, "flops": pairs}
+    if kind == "sparse":
+        kept = _kept(blocks, -(-_frame_tokens(case) // BLOCK))
+        return {"bytes": 4 * tensor + 4 * cells * kept, "flops": pairs * kept}
+    if kind == "update":
+        sampled = heads * blocks * SAMPLES
+        reads = 2 * sampled * HEAD_DIM * size + (cells if case["previous"] else 0)
+        return {"bytes": reads + cells * (4 + 1 + 4 * 0.625),
+                "flops": 2.0 * HEAD_DIM * sampled * blocks * SAMPLES}
+    if kind == "exact":
+        return {"bytes": 4 * tensor + 4 * rows + cells * (4 + 1 + 4 * 0.625), "flops": pairs}
+    if kind in ("tile", "boot"):
+        _, tiles, sink = _tile_counts(case)
+        kept = _kept(tiles, sink) if kind == "tile" else 1.0
+        cells = heads * tiles * tiles
+        # fp32 mass, fp16 mass, four fp16 centroids, the next route (and the old one).
+        per_cell = 4 + 2 + 4 * 2 + 1 + (1 if kind == "tile" else 0)
+        return {"bytes": 4 * tensor + 4 * rows + cells * per_cell, "flops": pairs * kept}
+    dim, ffn, layers = 1536, 8960, case["layers"]
+    gemm = 2.0 * tokens * (6 * dim * dim + 2 * dim * ffn) + 4.0 * TEXT_TOKENS * dim * dim
+    cross = 4.0 * HEAD_DIM * rows * TEXT_TOKENS
+    weights = 2 * (8 * dim * dim + 2 * dim * ffn)
+    # Per block: every weight once, the residual stream in and out.
+    return {"bytes": layers * (weights + 2 * tensor), "flops": layers * (gemm + cross + pairs)}
+
+
+def tolerance(case):
+    """About four times the distance measured between the path and `exact`
+    (2.3e-3 in bf16, 2.9e-4 in fp16, 7e-7 to 3e-6 in fp32, 4e-6 for the
+    sampled mass, 5e-3 for two bf16 DiT blocks) and, for whole values, between
+    two runs that walk the keys in another order (route cells at a threshold
+    fall on either side: 1e-3 of the row counts at 720p)."""
+    kind, dtype = case["kind"], case["dtype"]
+    rel = {"bf16": 1e-2, "fp16": 1.5e-3, "fp32": 1e-5}[dtype]
+    if kind in ("dense", "sparse"):
+        return {"rel": rel}
+    if kind == "dit":
+        return {"rel": 2e-2}
+    if kind == "update":
+        return {"rel": 2e-5, "max": 2e-2, "differ": 2e-3}
+    # The statistics' fp16 outputs (centroids, mass) set the floor of rel.
+    return {"rel": max(rel, 1.5e-3), "max": 0.1, "differ": 4e-3}
+
+
+# ---------------------------------------------------------------------------
+# The same results in 64 bits
+# ---------------------------------------------------------------------------
+
+def _attend(q, k, v, keep=None, unit=1, tile_shape=None, mass_unit=0):
+    """Softmax attention in float64 over [B, T, H, D] tensors.
+
+    keep: bool [H, units, units] of attended (query, key) units of `unit`
+    tokens.  Returns out, lse [B, H, T] and, with `tile_shape`, the mass and
+    moment sums of every (query tile, key tile) [5, H, tiles, tiles], or with
+    `mass_unit` the plain block mass [H, blocks, blocks]."""
+    batch, tokens, heads, dim = q.shape
+    out = torch.empty((batch, tokens, heads, dim), dtype=torch.float64, device=q.device)
+    lse = torch.empty((batch, heads, tokens), dtype=torch.float64, device=q.device)
+    sums = mass = None
+    if tile_shape is not None:
+        tiles = tokens // unit
+        sums = torch.zeros((5, heads, tiles, tiles), dtype=torch.float64, device=q.device)
+        y, x = (_axis(n) for n in tile_shape)
+        offsets = torch.stack((torch.ones(unit, dtype=torch.float64),
+                               y.repeat_interleave(tile_shape[1]), x.repeat(tile_shape[0])),
+                              dim=1).to(q.device)  # [unit, 3]
+    if mass_unit:
+        blocks = -(-tokens // mass_unit)
+        mass = torch.zeros((heads, blocks, blocks), dtype=torch.float64, device=q.device)
+    granule = unit if keep is not None or tile_shape is not None else (mass_unit or 1)
+    step = max(granule, (1 << 27) // k.shape[1] // granule * granule)
+    for b in range(batch):
+        for h in range(heads):
+            keys = k[b, :, h].double().t().contiguous()
+            values = v[b, :, h].double().contiguous()
+            for r0 in range(0, tokens, step):
+                r1 = min(tokens, r0 + step)
+                s = (q[b, r0:r1, h].double() * dim ** -0.5) @ keys
+                if keep is not None:
+                    rows = keep[h, r0 // unit:-(-r1 // unit)].repeat_interleave(unit, dim=0)
+                    cols = rows.repeat_interleave(unit, dim=1)[:r1 - r0, :k.shape[1]]
+                    s.masked_fill_(~cols, -math.inf)
+                    del cols
+                total = torch.logsumexp(s, dim=1)
+                s.sub_(total[:, None]).exp_()
+                lse[b, h, r0:r1] = total
+                out[b, r0:r1, h] = s @ values
+                if sums is not None:
+                    n = (r1 - r0) // unit
+                    part = s.view(n, unit, tiles, unit).reshape(-1, unit) @ offsets
+                    part = part.view(n, unit, tiles, 3)  # per row: 1, y, x of the key side
+                    at = slice(r0 // unit, r1 // unit)
+                    sums[0, h, at] = part[..., 0].sum(1)
+                    sums[1, h, at] = (part[..., 0] * offsets[None, :, None, 1]).sum(1)
+                    sums[2, h, at] = (part[..., 0] * offsets[None, :, None, 2]).sum(1)
+                    sums[3, h, at] = part[..., 1].sum(1)
+                    sums[4, h, at] = part[..., 2].sum(1)
+                if mass is not None:
+                    pad = F.pad(s, (0, blocks * mass_unit - tokens,
+                                    0, -(r1 - r0) % mass_unit))
+                    mass[h, r0 // mass_unit:-(-r1 // mass_unit)] = pad.view(
+                        -1, mass_unit, blocks, mass_unit).sum(dim=(1, 3))
+    return out, lse, sums if sums is not None else mass
+
+
+def _axis(n):
+    """Offsets of n positions on a tile side, scaled to [-1, 1]."""
+    center = (n - 1) / 2
+    return (torch.arange(n, dtype=torch.float64) - center) / max(center, 0.5)
+
+
+def _sampled_mass(case, q, k):
+    """Mean softmax mass per block pair of the sampled tokens; the scores are
+    a matmul and a scale multiply in the input type, as the path defines."""
+    tokens, heads, dtype = _shape(case)
+    blocks = -(-tokens // BLOCK)
+    first = torch.arange(blocks, device="cuda") * BLOCK
+    sizes = torch.clamp(tokens - first, max=BLOCK)
+    s = torch.arange(SAMPLES, device="cuda")
+    local = torch.minimum((2 * s + 1)[None] * sizes[:, None] // (2 * SAMPLES), sizes[:, None] - 1)
+    index = (first[:, None] + local).reshape(-1)
+    log_weight = torch.log(sizes.double() / SAMPLES).repeat_interleave(SAMPLES)
+    mass = torch.empty((heads, blocks, blocks), dtype=torch.float64, device="cuda")
+    scale = HEAD_DIM ** -0.5
+    for h in range(heads):
+        qs, ks = q[0, index, h].double(), k[0, index, h].double()
+        score = (qs @ ks.t().contiguous()).to(dtype)
+        score = (score.float() * scale).to(dtype).double() + log_weight
+        p = torch.softmax(score, dim=1)
+        mass[h] = p.view(blocks, SAMPLES, blocks, SAMPLES).sum(3).mean(1)
+    return mass
+
+
+def _dit(case, seed):
+    """The DiT's forward in float64 on the weights and inputs of `prepare`."""
+    state = prepare(case, seed)
+    model, config = state["model"], state["model"].config
+
+    def linear(x, wb):
+        return x @ wb[0].double().t().contiguous() + wb[1].double()
+
+    def norm(x):
+        return F.layer_norm(x, x.shape[-1:], eps=config.eps)
+
+    def rms(x, weight):
+        return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + config.eps) * weight.double()
+
+    grid = (case["frames"], case["height"], case["width"])
+    tokens, heads, dim = math.prod(grid), config.heads, config.dim
+    table = rope_cos_sin(grid, config.head_dim, device="cuda").double()
+    cos, sin = table[:, None, :, 0], table[:, None, :, 1]
+
+    def rope(x):
+        x = x.view(tokens, heads, config.head_dim)
+        a, b = x[..., 0::2], x[..., 1::2]
+        return torch.stack((a * cos - b * sin, a * sin + b * cos), dim=-1).reshape(
+            1, tokens, heads, config.head_dim)
+
+    latents = state["latents"][0].double()
+    patches = latents.view(config.in_channels, grid[0], grid[1], 2, grid[2], 2)
+    x = linear(patches.permute(1, 2, 4, 0, 3, 5).reshape(tokens, -1), model.patch)
+    half = config.freq_dim // 2
+    args = 882.0 * torch.exp(-math.log(10000.0) * torch.arange(half, dtype=torch.float64) / half)
+    t = torch.cat((torch.cos(args), torch.sin(args))).cuda()
+    temb = linear(F.silu(linear(t, model.time1)), model.time2)
+    temb6 = linear(F.silu(temb), model.time_proj).view(6, dim)
+    context = state["context"][0].double()
+    split = (1, -1, heads, config.head_dim)
+    for block in model.blocks:
+        mod = block["table"].double() + temb6
+        h = norm(x) * (1 + mod[1]) + mod[0]
+        q = rope(rms(linear(h, block["q"]), block["norm_q"]))
+        k = rope(rms(linear(h, block["k"]), block["norm_k"]))
+        out = _attend(q, k, linear(h, block["v"]).view(split))[0]
+        x = x + mod[2] * linear(out.view(tokens, dim), block["o"])
+        h = norm(x) * block["norm2_w"].double() + block["norm2_b"].double()
+        q = rms(linear(h, block["cq"]), block["cnorm_q"]).view(split)
+        k = rms(linear(context, block["ck"]), block["cnorm_k"]).view(split)
+        out = _attend(q, k, linear(context, block["cv"]).view(split))[0]
+        x = x + linear(out.view(tokens, dim), block["co"])
+        h = norm(x) * (1 + mod[4]) + mod[3]
+        x = x + mod[5] * linear(F.gelu(linear(h, block["ffn1"]), approximate="tanh"),
+                                block["ffn2"])
+    shift, scale = model.head_table.double() + temb
+    out = linear(norm(x) * (1 + scale) + shift, model.head)
+    out = out.view(1, *grid, config.out_channels, 1, 2, 2)
+    return out.permute(0, 4, 1, 5, 2, 6, 3, 7).reshape(state["latents"].shape)
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "dit":
+        return _dit(case, seed)
+    state = prepare(case, seed)
+    q, k, v = state["q"], state["k"], state["v"]
+    tokens = q.shape[1]
+    if kind == "dense":
+        return _attend(q, k, v)[0]
+    if kind == "sparse":
+        layout = state.get("layout")
+        if layout is not None:
+            order = layout.permutation_cpu.long().cuda()
+            q, k, v = q[:, order], k[:, order], v[:, order]
+        out = _attend(q, k, v, state["csr"].to_route().reshape(
+            q.shape[2], -1, -(-tokens // BLOCK)), BLOCK)[0]
+        return out if layout is None else out[:, layout.inverse_cpu.long().cuda()]
+    if kind == "update":
+        return {"mass": _sampled_mass(case, q, k), "route": None, "counts": None,
+                "row_ptr": None}
+    if kind == "exact":
+        out, lse, mass = _attend(q, k, v, mass_unit=BLOCK)
+        return {"out": out, "lse": lse, "mass": mass, "route": None, "counts": None,
+                "row_ptr": None}
+    tile = case["tile_h"] * case["tile_w"]
+    keep = state.get("route")
+    out, lse, sums = _attend(q, k, v, keep, tile, (case["tile_h"], case["tile_w"]))
+    mass = sums[0] / tokens
+    den = sums[0].clamp_min(1e-12)
+    return {"out": out, "lse": lse, "route": None, "counts": None, "mass": mass,
+            "mass_f16": mass, "centroid_q_y": sums[1] / den, "centroid_q_x": sums[2] / den,
+            "centroid_k_y": sums[3] / den, "centroid_k_x": sums[4] / den}
