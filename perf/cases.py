@@ -337,8 +337,9 @@ def tolerance(case):
         return {"rel": 2e-2}
     if kind == "update":
         return {"rel": 2e-5, "max": 2e-2, "differ": 2e-3}
-    # The statistics' fp16 outputs (centroids, mass) set the floor of rel.
-    return {"rel": max(rel, 1.5e-3), "max": 0.1, "differ": 4e-3}
+    # In float32 the fp16 outputs (centroids, mass) set the floor: a value at a
+    # rounding boundary may land one fp16 step away.
+    return {"rel": max(rel, 1e-4), "max": 0.1, "differ": 4e-3}
 
 
 # ---------------------------------------------------------------------------
