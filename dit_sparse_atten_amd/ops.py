@@ -309,10 +309,10 @@ def bsa_fwd_block_mass(q, k, v, scale=None):
     ``lse`` [1, H, T] as :func:`bsa_fwd` returns them and ``mass`` as
     :func:`block_mass` does (the reference's ``_dense_bootstrap`` pair of
     dense attention and ``_block_attention_mass``, attention_backends/
-    flex.py:254-272, 158-202).  With T a multiple of 128 the mass comes from
-    the attention launch's own probabilities; otherwise the call runs the
-    attention and then the block-mass pass (bf16 and fp16; float32 inputs
-    need T a multiple of 128).
+    flex.py:254-272, 158-202).  The mass comes from the attention launch's own
+    probabilities; only head dims above 128 with T not a multiple of 128 run
+    the attention and then the block-mass pass.  float32 inputs need T a
+    multiple of 128.
     """
     lib = _lib.load()
     q = _kernel_view("q", q, attention=True)

@@ -88,6 +88,25 @@ def test_dense_with_block_mass_matches_oracle(ops, cuda_device, tokens):
                                np.broadcast_to(valid, mass.shape[:2]), rtol=2e-4)
 
 
+@pytest.mark.parametrize("tokens,heads,dtype", [
+    (1, 1, torch.bfloat16), (127, 2, torch.float16), (129, 2, torch.bfloat16),
+    (191, 3, torch.float16), (2100, 40, torch.bfloat16)])
+def test_block_mass_of_a_partial_last_block(ops, cuda_device, tokens, heads, dtype):
+    """The fused block mass with a partial last block of 1, 127, 1, 63 and 52
+    tokens (one wave, a partial and an empty half-tile; 680 workgroups with a
+    split last round at 2,100 tokens), against the fp64 mass of the same LSE.
+    fp32 sums of exactly the attention's exp2 values: MASS_RTOL."""
+    q, k, v = clustered_qkv(tokens, heads, 128, group=64, seed=tokens, dtype=dtype)
+    qd, kd, vd = (x.to(cuda_device) for x in (q, k, v))
+    out, lse, mass = ops.bsa_fwd_block_mass(qd, kd, vd)
+    ref_out, ref_lse = ops.bsa_fwd(qd, kd, vd, return_lse=True)
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(lse.cpu().numpy(), ref_lse.cpu().numpy(), atol=LSE_ATOL)
+    assert (out.float() - ref_out.float()).abs().max().item() <= 8e-3
+    expected = E.exact_block_mass(q.float().numpy(), k.float().numpy(), lse[0].cpu().numpy(), 128)
+    np.testing.assert_allclose(mass.cpu().numpy(), expected, rtol=MASS_RTOL, atol=MASS_ATOL)
+
+
 def test_block_mass_explicit_softmax_reference_test(ops, cuda_device):
     """tests/test_flex_backend.py:78-99 at head_dim 128: 250 tokens, 2 heads;
     LSE from an fp32 logsumexp rather than the attention kernel."""
