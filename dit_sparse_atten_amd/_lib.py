@@ -68,6 +68,15 @@ SIGNATURES = {
         _c_int, _c_int, _c_int, _c_int, _c_int,    # tokens, heads, head_dim, block, samples
         _c_float, _c_ptr, _c_ptr,                  # scale, mass, stream
     )),
+    "dsa_sampled_mass_ws": (_c_int, (
+        _c_ptr, _c_ptr, _c_int,                    # q, k, dtype
+        ctypes.POINTER(_c_i64),                    # strides[4]
+        _c_int, _c_int, _c_int, _c_int, _c_int,    # tokens, heads, head_dim, block, samples
+        _c_float, _c_ptr, _c_ptr, _c_size, _c_ptr,  # scale, mass, workspace, bytes, stream
+    )),
+    "dsa_sampled_mass_workspace_bytes": (_c_size, (
+        _c_int, _c_int, _c_int, _c_int,            # tokens, heads, block, samples
+    )),
     "dsa_block_mass": (_c_int, (
         _c_ptr, _c_ptr, _c_int,                    # q, k, dtype
         ctypes.POINTER(_c_i64),                    # strides[4]

@@ -18,6 +18,7 @@
 // block sum goes through LDS and the workgroup adds them in a fixed order
 // after the next barrier (no atomics: the mass, the input of the bit-exact
 // route selection, is run-to-run deterministic).
+#include <algorithm>
 #include <type_traits>
 
 #include "bsa_tiles.h"
@@ -37,7 +38,22 @@ struct MassParams {
   float scale;      // score scale (d^-1/2 unless given)
   float logw_full;  // log(block_size / S)
   float logw_last;  // log(size of the last block / S)
+  // One-sweep kernel: row-block sums of the launch's workgroups (kRowSlot
+  // floats per key block and workgroup), and the launch's first workgroup.
+  float* part;
+  int32_t first, row_tiles;  // row_tiles: 128-row workgroups per head
 };
+
+constexpr int kGroupRows = 128;  // sampled query rows per workgroup
+// The one-sweep kernel moves a row's reference once a sub-tile adds more than
+// this to it: a row sum of up to 2^20 sub-tiles then stays finite.
+constexpr float kMoveSum = 1152921504606846976.0f;  // 2^60
+
+// Key blocks per slot of row sums: whole 64-key tiles of any sample count, so
+// that every sub-tile stores its sums without a bound check.
+__host__ __device__ constexpr int64_t part_blocks(int64_t blocks) {
+  return (blocks + 63) / 64 * 64;
+}
 
 // Token of padded sample slot j (block j / SP, sample j % SP) for S real
 // samples per block (flex.py:224-231); a padding slot repeats the block's
@@ -70,24 +86,36 @@ __device__ __forceinline__ void round_pair(float a, float b, float& ra, float& r
   }
 }
 
-// One workgroup (4 waves x 32 sampled queries) scans every sampled key twice:
-// sweep 1 builds each query's log-sum-exp, sweep 2 sums the normalised
-// probabilities per (query block, key block).  The sampled score matrix is
-// never written to memory.  The scan is VALU-bound (the per-score rounding
-// and softmax work outweighs the 32x32x16 MFMAs several times), so scores
-// are rounded in pairs, the log2(e) scale and log-weight fold into one fma,
-// the max runs over the rounded scores, and only the tile holding the
-// sequence's last sampled keys (every tile with padding slots) pays the
-// per-score checks.  Sampled key rows are gathered straight into LDS (buffer
-// loads with a per-lane row offset), double-buffered one 64-key tile ahead.
+// One workgroup (4 waves x 32 sampled queries) scans every sampled key; the
+// sampled score matrix is never written to memory.  The scan is VALU-bound
+// (the per-score rounding and softmax work outweighs the 32x32x16 MFMAs
+// several times), so scores are rounded in pairs, the log2(e) scale and
+// log-weight fold into one fma, and only the tile holding the sequence's last
+// sampled keys (every tile with padding slots) pays the per-score checks.
+// Sampled key rows are gathered straight into LDS (buffer loads with a
+// per-lane row offset), double-buffered one 64-key tile ahead.
+//
+// kOnce: one sweep.  Each query row keeps its scores' reference fixed (the
+// largest score of its first sub-tile; fp32's exponent range absorbs what
+// later scores exceed it by, and a row moves its reference, and rescales what
+// it has written, only past kMoveSum), writes the sum of its terms per key
+// block to p.part and, after the scan, reads them back and adds the rows of
+// each query block over their row totals.  Writing and reading 4 bytes per
+// (row, key block) costs far less than the second sweep's rounding, fma, exp
+// and add per score: 57,600 tokens x 40 heads, 16 samples, same
+// box: 1.02 against 1.73 ms.  Without a workspace (kOnce = false; also SP >= 64, whose blocks
+// span waves) sweep 1 builds each query's log-sum-exp and sweep 2 sums the
+// normalised probabilities per (query block, key block).  Three waves per SIMD
+// (168 VGPRs): with four, the longer instances spill.
 //
 // kHalves: head dims up to 128 * kHalves.  Head dims above 128 stage each
 // tile as two 128-dim halves (dims 0..127, then 128..) and add both halves'
 // products into one fp32 accumulator before the score is rounded, as one
 // matmul over all dims does.
-template <typename T, int SP, bool kPad, int kHalves = 1>
-__global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
+template <typename T, int SP, bool kPad, int kHalves, bool kOnce>
+__global__ void __launch_bounds__(256, kHalves == 1 ? 3 : 2) sampled_mass_kernel(MassParams p) {
   typedef dsa::Elem<T> E;
+  static_assert(!kOnce || SP <= 32, "one sweep: query blocks within a wave");
   constexpr int kTileKeys = 64;
   constexpr int kHalfBytes = kTileKeys * 256;  // one 128-dim half of a tile
   constexpr bool kWide = SP >= 64;
@@ -101,11 +129,13 @@ __global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5;
   const int qi = lane & 31;
-  const int h = blockIdx.y;
+  const int group = p.first + (int)blockIdx.x;
+  const int h = group / p.row_tiles;
+  const int row0 = (group % p.row_tiles) * kGroupRows;
   const int S = kPad ? p.samples : SP;
   const int ns = p.blocks * SP;
   const int tiles = (ns + kTileKeys - 1) / kTileKeys;
-  const int q0 = blockIdx.x * 128 + wave * 32;  // first sampled query of this wave
+  const int q0 = row0 + wave * 32;  // first sampled query of this wave
 
   int qs = q0 + qi;
   const bool q_real = qs < ns && (qs % SP) < S;
@@ -124,10 +154,46 @@ __global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
   for (int hf = 0; hf < kHalves; ++hf)
     k_rsrc[hf] = dsa::make_rsrc(kbase + 128 * hf,
                                 (uint32_t)(((int64_t)(p.tokens - 1) * p.k_st + kHeadDim) * 2));
+  const int last_block = p.blocks - 1;
+  // Tiles before this one hold only full, in-range key blocks.
+  const int first_tail_tile = (last_block * SP) / kTileKeys;
   // This lane's 4 chunks of tile t: LDS slot idx = (wave * 4 + j) * 64 + lane
-  // holds chunk (idx & 15) ^ (row & 15) of tile row idx >> 4.
+  // holds chunk (idx & 15) ^ (row & 15) of tile row idx >> 4.  In a tile of
+  // full blocks the row's token is that of tile 0 plus 64 / SP blocks per tile
+  // (SP <= 64), so its offset is a per-lane constant plus a uniform one: the
+  // general form (a division and a 64-bit multiply per chunk) took a fifth of
+  // the scan's VALU work.
+  constexpr bool kTileBlocks = SP <= kTileKeys;
+  const uint32_t tile_step =
+      (uint32_t)((int64_t)(kTileKeys / SP) * p.block_size * p.k_st * 2);
+  uint32_t chunk_at[4];
+  if constexpr (kTileBlocks) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int idx = (wave * 4 + j) * 64 + lane;
+      const int row = idx >> 4;
+      const int c = (idx & 15) ^ (row & 15);
+      // (Blocks past a one-block sequence: those tiles take the general form.)
+      const int s = row % SP < S ? row % SP : S - 1;
+      const int token = row / SP * p.block_size + ((2 * s + 1) * p.block_size) / (2 * S);
+      chunk_at[j] = (uint32_t)(((int64_t)token * p.k_st + c * 8) * 2);
+    }
+  }
   auto issue = [&](int t, unsigned char* dst) __attribute__((always_inline)) {
     const int kt0 = t * kTileKeys;
+    if (kTileBlocks && t < first_tail_tile) {
+      const uint32_t at = (uint32_t)t * tile_step;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int idx = (wave * 4 + j) * 64 + lane;
+        const int c = (idx & 15) ^ ((idx >> 4) & 15);
+#pragma unroll
+        for (int hf = 0; hf < kHalves; ++hf)
+          dsa::lds_load16(k_rsrc[hf], dst + hf * kHalfBytes + (wave * 4 + j) * 1024,
+                          (chunk_at[j] + at) | dsa::dead_bits(c, p.head_dim - 128 * hf), 0);
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int idx = (wave * 4 + j) * 64 + lane;
@@ -144,17 +210,25 @@ __global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
     }
   };
 
-  const int last_block = p.blocks - 1;
   const float c_full = p.logw_full * kLog2e;
   const float c_last = p.logw_last * kLog2e;
-  // Tiles before this one hold only full, in-range key blocks.
-  const int first_tail_tile = kPad ? 0 : (last_block * SP) / kTileKeys;
   float m2 = -INFINITY, l2 = 0.f, lse2 = 0.f;
   float wide_acc = 0.f;  // kWide: this lane's sum over the current key block
+  // kOnce: this wave's row sums [key block][32 rows].
+  float* const part =
+      kOnce ? p.part + ((int64_t)blockIdx.x * 4 + wave) * 32 * part_blocks(p.blocks) : nullptr;
+  // Makes the wave's own stores to `part` visible to its loads.
+  auto settle_part = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  };
 
-  auto compute = [&](const unsigned char* lds_k, int t, int sweep) __attribute__((always_inline)) {
+  // One tile; kTail: it may hold keys of the last block, padding slots or
+  // slots past the end.
+  auto compute_tile = [&](const unsigned char* lds_k, int t, int sweep, auto tail_c)
+      __attribute__((always_inline)) {
+    constexpr bool kTail = decltype(tail_c)::value;
     const int kt0 = t * kTileKeys;
-    const bool tail = t >= first_tail_tile;
 #pragma unroll
     for (int sub = 0; sub < kTileKeys / 32; ++sub) {
       dsa_f32x16 acc;
@@ -173,29 +247,102 @@ __global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
       // Score = T(T(q.k) * scale), as a matmul and a scale multiply in T;
       // the softmax input in log2 units is score * log2e + c with
       // c = log(block size / S) * log2e.
-      float sc[16], cw[16];
+      float sc[16];
+      [[maybe_unused]] float cws[16];
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
         float a0, a1;
         round_pair<T>(acc[r], acc[r + 1], a0, a1);
         round_pair<T>(a0 * p.scale, a1 * p.scale, sc[r], sc[r + 1]);
       }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) cw[r] = c_full;
-      if (tail) {
+      if constexpr (kTail) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int j = kt0 + sub * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-          cw[r] = j / SP == last_block ? c_last : c_full;
+          cws[r] = j / SP == last_block ? c_last : c_full;
           if (j >= ns || (kPad && (j % SP) >= S)) sc[r] = -INFINITY;
         }
       }
-      if (sweep == 0) {
+      auto cw = [&](int r) __attribute__((always_inline)) {
+        if constexpr (kTail) return cws[r];
+        else return c_full;
+      };
+      if constexpr (kOnce) {
+        // Key-block sums of this lane: key 8 (r >> 2) + 4 g + (r & 3) of the
+        // sub-tile.  Blocks of 8 or more samples hold keys of both lane
+        // halves (sum i: block i), shorter ones of one half (sum i: the block
+        // of accumulator i SP).
+        constexpr int kOwn = SP >= 8 ? 32 / SP : 16 / SP;
+        const int kb0 = (kt0 + sub * 32) / SP;
+        // (The empty asm keeps the compiler from computing it ahead of the
+        // branches that need it, on every sub-tile.)
+        auto row_max = [&]() __attribute__((always_inline)) {
+          float log2e = kLog2e;
+          asm volatile("" : "+v"(log2e));
+          float mx = -INFINITY;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fmaf(sc[r], log2e, cw(r)));
+          return dsa::pair32_max(mx);
+        };
+        // The reference: the largest score of the row's first sub-tile that
+        // has one above -inf (0 until then, when every term is 0).
+        if (__any(m2 == -INFINITY)) {
+          const float mx = row_max();
+          if (m2 == -INFINITY) m2 = mx;
+        }
+        float pk[kOwn];
+        auto terms = [&]() __attribute__((always_inline)) {
+          const float mref = m2 == -INFINITY ? 0.f : m2;
+#pragma unroll
+          for (int i = 0; i < kOwn; ++i) pk[i] = 0.f;
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            pk[(SP >= 8 ? 8 * (r >> 2) : r) / SP] +=
+                __builtin_amdgcn_exp2f(fmaf(sc[r], kLog2e, cw(r) - mref));
+          float sum = 0.f;
+#pragma unroll
+          for (int i = 0; i < kOwn; ++i) sum += pk[i];
+          return sum;
+        };
+        float sum = terms();
+        if (__any(!(sum <= kMoveSum))) {
+          // Some row's terms have outgrown its reference (or are not finite):
+          // move the reference to the row's largest score.
+          const float mx = row_max();
+          const bool up = mx > m2;
+          const float alpha = up ? __builtin_amdgcn_exp2f(m2 - mx) : 1.f;
+          if (up) m2 = mx;
+          l2 *= alpha;
+          settle_part();
+          for (int kb = g; kb < kb0; kb += 2) part[kb * 32 + qi] *= alpha;
+          settle_part();
+          sum = terms();
+        }
+        l2 += sum;
+        if constexpr (SP >= 8 && kOwn > 1) {
+          // Lane half g takes block i + g: the sum over both halves' keys.
+#pragma unroll
+          for (int i = 0; i < kOwn; i += 2) {
+            const auto both = __builtin_amdgcn_permlane32_swap(
+                __float_as_uint(pk[i]), __float_as_uint(pk[i + 1]), false, false);
+            part[(kb0 + i + g) * 32 + qi] = __uint_as_float(both[0]) + __uint_as_float(both[1]);
+          }
+        } else if constexpr (SP >= 8) {
+          const float total = dsa::pair32_sum(pk[0]);
+          if (g == 0) part[kb0 * 32 + qi] = total;
+        } else {
+#pragma unroll
+          for (int i = 0; i < kOwn; ++i) {
+            const int r = i * SP;
+            part[(kb0 + (8 * (r >> 2) + 4 * g + (r & 3)) / SP) * 32 + qi] = pk[i];
+          }
+        }
+      } else if (sweep == 0) {
         // Running max of x = score * log2e + c (log2e > 0: c_last differs
         // from c_full only in the tail).
         float mx = m2;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fmaf(sc[r], kLog2e, cw[r]));
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, fmaf(sc[r], kLog2e, cw(r)));
         // While every key this lane has seen is masked (mx = -inf, as for
         // the lanes past the last sampled key when blocks * S <= 4), the
         // terms and the rescale take a finite reference and are exactly
@@ -204,14 +351,14 @@ __global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
         float sum = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          sum += __builtin_amdgcn_exp2f(fmaf(sc[r], kLog2e, cw[r] - mref));
+          sum += __builtin_amdgcn_exp2f(fmaf(sc[r], kLog2e, cw(r) - mref));
         l2 = l2 * __builtin_amdgcn_exp2f(m2 - mref) + sum;
         m2 = mx;
       } else if constexpr (kWide) {
         float sum = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          sum += __builtin_amdgcn_exp2f(fmaf(sc[r], kLog2e, cw[r] - lse2));
+          sum += __builtin_amdgcn_exp2f(fmaf(sc[r], kLog2e, cw(r) - lse2));
         wide_acc += q_real ? sum : 0.f;
       } else {
         float pk[KBS];
@@ -220,7 +367,7 @@ __global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int local = 8 * (r >> 2) + 4 * g + (r & 3);
-          pk[local / SP] += __builtin_amdgcn_exp2f(fmaf(sc[r], kLog2e, cw[r] - lse2));
+          pk[local / SP] += __builtin_amdgcn_exp2f(fmaf(sc[r], kLog2e, cw(r) - lse2));
         }
         // Sum over the SP query lanes of each query block (padding lanes
         // add zero) and both halves.
@@ -254,6 +401,12 @@ __global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
       }
     }
   };
+  auto compute = [&](const unsigned char* lds_k, int t, int sweep) __attribute__((always_inline)) {
+    if (kPad || t >= first_tail_tile)
+      compute_tile(lds_k, t, sweep, std::bool_constant<true>{});
+    else
+      compute_tile(lds_k, t, sweep, std::bool_constant<false>{});
+  };
 
   // kWide: writes the mass of key block kb from the wave sums published for
   // it (after a barrier); the waves of one query block are added in order.
@@ -261,7 +414,7 @@ __global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
     if constexpr (kWide) {
       constexpr int kWavesPerBlock = SP / 32;
       if (tid < 4 / kWavesPerBlock) {
-        const int qb = (blockIdx.x * 128) / SP + tid;
+        const int qb = row0 / SP + tid;
         if (qb < p.blocks && kb < p.blocks) {
           float total = 0.f;
 #pragma unroll
@@ -279,21 +432,27 @@ __global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
   // the current one.
   auto step = [&](int t, int sweep, int next_t, const unsigned char* cur,
                   unsigned char* nxt) __attribute__((always_inline)) {
-    __builtin_amdgcn_s_waitcnt(kWide ? 0x0070 : 0x0F70);  // vmcnt(0) [lgkmcnt(0)]
+    // kOnce: the row sums of the previous tile, stored after the current
+    // tile's loads were issued, may still be on their way.
+    constexpr int kStores = !kOnce ? 0 : 2 * (SP >= 8 ? (SP == 32 ? 1 : 16 / SP) : 16 / SP);
+    if (kOnce && t > 0)
+      __builtin_amdgcn_s_waitcnt(0x0F70 | (kStores & 15) | ((kStores >> 4) << 14));  // vmcnt
+    else
+      __builtin_amdgcn_s_waitcnt(kWide ? 0x0070 : 0x0F70);  // vmcnt(0) [lgkmcnt(0)]
     __syncthreads();
     if (next_t >= 0) issue(next_t, nxt);
     if (kWide && sweep == 1 && t > 0 && (t * kTileKeys) % SP == 0) flush_wide(t * kTileKeys / SP - 1);
     compute(cur, t, sweep);
   };
 
-  for (int sweep = 0; sweep < 2; ++sweep) {
+  for (int sweep = 0; sweep < (kOnce ? 1 : 2); ++sweep) {
     issue(0, st0);
     for (int t = 0; t < tiles; t += 2) {
       step(t, sweep, t + 1 < tiles ? t + 1 : -1, st0, st1);
       if (t + 1 >= tiles) break;
       step(t + 1, sweep, t + 2 < tiles ? t + 2 : -1, st1, st0);
     }
-    if (sweep == 0) {  // each query's log-sum-exp (log2 units)
+    if (!kOnce && sweep == 0) {  // each query's log-sum-exp (log2 units)
       // Lanes l and l ^ 32 hold the two halves of one query's keys; both get
       // the same total (the pair's two terms in one fixed order, so a
       // contracted fma rounds alike in both lanes).
@@ -313,14 +472,62 @@ __global__ void __launch_bounds__(256) sampled_mass_kernel(MassParams p) {
     dsa::lds_barrier();
     flush_wide(p.blocks - 1);
   }
+  if constexpr (kOnce) {
+    // mass[qb][kb] = sum over the rows of qb of part[kb][row] / total[row] / S.
+    // Eight lanes read one key block's 32 rows (four each), so a wave reads
+    // 1 KB of consecutive part per step.
+    settle_part();
+    const float total = dsa::pair32_sum(l2);
+    const float weight = q_real ? 1.f / total : 0.f;
+    const int sub_rows = lane & 7;
+    float w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = __shfl(weight, 4 * sub_rows + i);
+    constexpr int kLanes = SP >= 4 ? SP / 4 : 1;  // lanes per query block
+    constexpr int kVals = SP >= 4 ? 1 : 4 / SP;   // query blocks per lane
+    constexpr int kAhead = 4;                     // loads in flight per lane
+    for (int k0 = lane >> 3; k0 - (lane >> 3) < p.blocks; k0 += 8 * kAhead) {
+      dsa_f32x4 x[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int kb = k0 + 8 * u;
+        x[u] = kb < p.blocks
+                   ? *reinterpret_cast<const dsa_f32x4*>(part + kb * 32 + 4 * sub_rows)
+                   : dsa_f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int kb = k0 + 8 * u;
+        float val[kVals];
+#pragma unroll
+        for (int v = 0; v < kVals; ++v) {
+          val[v] = 0.f;
+#pragma unroll
+          for (int i = 0; i < 4 / kVals; ++i)
+            val[v] = fmaf(x[u][v * (4 / kVals) + i], w[v * (4 / kVals) + i], val[v]);
+        }
+#pragma unroll
+        for (int m = 1; m < kLanes; m <<= 1) val[0] += __shfl_xor(val[0], m);
+        if (kb < p.blocks && sub_rows % kLanes == 0) {
+#pragma unroll
+          for (int v = 0; v < kVals; ++v) {
+            const int qb = q0 / SP + sub_rows / kLanes * kVals + v;
+            if (qb < p.blocks)
+              p.mass[((int64_t)h * p.blocks + qb) * p.blocks + kb] = val[v] / (float)S;
+          }
+        }
+      }
+    }
+  }
 }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
 
-template <typename T, int kHalves>
-void launch_mass(const MassParams& p, int sp, bool pad, dim3 grid, hipStream_t stream) {
-#define DSA_MASS(SPV, PADV) \
-  hipLaunchKernelGGL((sampled_mass_kernel<T, SPV, PADV, kHalves>), grid, dim3(256), 0, stream, p)
+template <typename T, int kHalves, bool kOnce>
+void launch_mass(const MassParams& p, int sp, bool pad, int groups, hipStream_t stream) {
+#define DSA_MASS(SPV, PADV)                                                           \
+  hipLaunchKernelGGL((sampled_mass_kernel<T, SPV, PADV, kHalves, kOnce>),             \
+                     dim3((unsigned)groups), dim3(256), 0, stream, p)
   if (!pad) {
     switch (sp) {
       case 1: DSA_MASS(1, false); break;
@@ -336,19 +543,71 @@ void launch_mass(const MassParams& p, int sp, bool pad, dim3 grid, hipStream_t s
       case 8: DSA_MASS(8, true); break;
       case 16: DSA_MASS(16, true); break;
       case 32: DSA_MASS(32, true); break;
-      case 64: DSA_MASS(64, true); break;
-      default: DSA_MASS(128, true); break;
+      case 64: if constexpr (!kOnce) DSA_MASS(64, true); break;
+      default: if constexpr (!kOnce) DSA_MASS(128, true); break;
     }
   }
 #undef DSA_MASS
 }
 
+template <typename T>
+void launch_mass(const MassParams& p, int sp, bool pad, bool once, int groups,
+                 hipStream_t stream) {
+  if (p.head_dim > kHeadDim)
+    once ? launch_mass<T, 2, true>(p, sp, pad, groups, stream)
+         : launch_mass<T, 2, false>(p, sp, pad, groups, stream);
+  else
+    once ? launch_mass<T, 1, true>(p, sp, pad, groups, stream)
+         : launch_mass<T, 1, false>(p, sp, pad, groups, stream);
+}
+
+// Power-of-two sample stride of S samples per block.
+int sample_stride(int32_t samples) {
+  int sp = 1;
+  while (sp < samples) sp <<= 1;
+  return sp;
+}
+
+// One-sweep workspace: a slot of row sums per workgroup, for the smaller of
+// every workgroup and kMinSlots or what kSlotBytes holds; larger calls run in
+// several launches over the same slots.  kMinSlots is what the chip holds at
+// once (four workgroups of 32 KB LDS per CU), so a launch of fewer would idle
+// CUs.
+constexpr int64_t kMinSlots = 1024;
+constexpr int64_t kSlotBytes = (int64_t)1 << 30;
+
+int64_t slot_bytes(int64_t blocks) {
+  return part_blocks(blocks) * kGroupRows * (int64_t)sizeof(float);
+}
+
 }  // namespace
+
+extern "C" size_t dsa_sampled_mass_workspace_bytes(int32_t tokens, int32_t heads,
+                                                   int32_t block_size, int32_t samples) {
+  if (tokens <= 0 || heads <= 0 || block_size <= 0 || block_size > 128 || samples <= 0 ||
+      samples > block_size)
+    return 0;
+  const int sp = sample_stride(samples);
+  if (sp > 32) return 0;
+  const int64_t blocks = ((int64_t)tokens + block_size - 1) / block_size;
+  const int64_t groups = (blocks * sp + kGroupRows - 1) / kGroupRows * heads;
+  const int64_t slots = std::max(kMinSlots, kSlotBytes / slot_bytes(blocks));
+  return (size_t)(std::min(groups, slots) * slot_bytes(blocks));
+}
 
 extern "C" int dsa_sampled_mass(const void* q, const void* k, int32_t dtype,
                                 const int64_t* strides, int32_t tokens, int32_t heads,
                                 int32_t head_dim, int32_t block_size, int32_t samples,
                                 float scale, float* mass, hipStream_t stream) {
+  return dsa_sampled_mass_ws(q, k, dtype, strides, tokens, heads, head_dim, block_size, samples,
+                             scale, mass, nullptr, 0, stream);
+}
+
+extern "C" int dsa_sampled_mass_ws(const void* q, const void* k, int32_t dtype,
+                                   const int64_t* strides, int32_t tokens, int32_t heads,
+                                   int32_t head_dim, int32_t block_size, int32_t samples,
+                                   float scale, float* mass, void* workspace,
+                                   size_t workspace_bytes, hipStream_t stream) {
   dsa::clear_error();
   if (!q || !k || !mass || !strides)
     return dsa::set_error(DSA_EINVAL, "dsa_sampled_mass: null pointer");
@@ -376,8 +635,9 @@ extern "C" int dsa_sampled_mass(const void* q, const void* k, int32_t dtype,
   if (((int64_t)(tokens - 1) * strides[2] + kHeadDim) * 2 > 0x7fffffff)
     return dsa::set_error(DSA_EUNSUPPORTED,
                           "dsa_sampled_mass: one head's K rows must span < 2 GiB");
-  int sp = 1;
-  while (sp < samples) sp <<= 1;  // power-of-two sample stride
+  if (workspace_bytes > 0 && (!workspace || !aligned16(workspace)))
+    return dsa::set_error(DSA_EINVAL, "dsa_sampled_mass: workspace must be 16-byte aligned");
+  const int sp = sample_stride(samples);
   MassParams p;
   p.q = q;
   p.k = k;
@@ -397,16 +657,24 @@ extern "C" int dsa_sampled_mass(const void* q, const void* k, int32_t dtype,
   p.logw_full = logf((float)block_size / (float)samples);
   p.logw_last = logf((float)last / (float)samples);
   const int ns = p.blocks * sp;
-  const dim3 grid((unsigned)((ns + 127) / 128), (unsigned)heads);
+  p.row_tiles = (ns + kGroupRows - 1) / kGroupRows;
+  const int64_t groups = (int64_t)p.row_tiles * heads;
+  if (groups > 0x7fffffff)
+    return dsa::set_error(DSA_EINVAL, "dsa_sampled_mass: grid too large");
   // Padded instances for sample counts that are not a power of two, and for
   // 64 and 128 samples (key and query blocks wider than a sub-tile or wave).
   const bool pad = sp != samples || sp > 32;
-  const bool wide = head_dim > kHeadDim;
-  if (dtype == DSA_F16)
-    wide ? launch_mass<_Float16, 2>(p, sp, pad, grid, stream)
-         : launch_mass<_Float16, 1>(p, sp, pad, grid, stream);
-  else
-    wide ? launch_mass<__bf16, 2>(p, sp, pad, grid, stream)
-         : launch_mass<__bf16, 1>(p, sp, pad, grid, stream);
+  // One sweep where the workspace holds a chip's worth of row sums.
+  const int64_t slots = std::min<int64_t>(
+      groups, workspace ? (int64_t)workspace_bytes / slot_bytes(p.blocks) : 0);
+  const bool once = sp <= 32 && slots >= std::min(groups, kMinSlots);
+  p.part = once ? static_cast<float*>(workspace) : nullptr;
+  const int64_t step = once ? slots : groups;
+  for (int64_t first = 0; first < groups; first += step) {
+    p.first = (int32_t)first;
+    const int n = (int)std::min(step, groups - first);
+    if (dtype == DSA_F16) launch_mass<_Float16>(p, sp, pad, once, n, stream);
+    else launch_mass<__bf16>(p, sp, pad, once, n, stream);
+  }
   return dsa::check_launch("dsa_sampled_mass");
 }

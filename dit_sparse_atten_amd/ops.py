@@ -253,10 +253,16 @@ def sampled_block_mass(q, k, block_size, samples=2, scale=None):
     blocks = math.ceil(tokens / block_size)
     mass = torch.empty((heads, blocks, blocks), dtype=torch.float32, device=q.device)
     strides = _lib.int64_array([q.stride(1), q.stride(2), k.stride(1), k.stride(2)])
+    # Row sums of a single scan (none above 32 samples, which scan twice).
+    workspace_bytes = lib.dsa_sampled_mass_workspace_bytes(tokens, heads, block_size, samples)
+    workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device)
+                 if workspace_bytes else None)
     with torch.cuda.device(q.device):
-        status = lib.dsa_sampled_mass(
+        status = lib.dsa_sampled_mass_ws(
             q.data_ptr(), k.data_ptr(), dtype_code(q.dtype), strides, tokens, heads, head_dim, block_size,
-            samples, float(scale), mass.data_ptr(), _stream_handle(q.device))
+            samples, float(scale), mass.data_ptr(),
+            workspace.data_ptr() if workspace is not None else None, workspace_bytes,
+            _stream_handle(q.device))
     _lib.check(status, "dsa_sampled_mass")
     return mass
 

@@ -188,6 +188,18 @@ int dsa_sampled_mass(const void* q, const void* k, int32_t dtype, const int64_t*
                      int32_t samples, float scale, float* mass, hipStream_t stream);
 
 /*
+ * dsa_sampled_mass with a workspace, 16-byte aligned: with at least
+ * dsa_sampled_mass_workspace_bytes(...) bytes (0 above 32 samples) every score
+ * is computed once instead of twice.  NULL and 0 are allowed.
+ */
+int dsa_sampled_mass_ws(const void* q, const void* k, int32_t dtype, const int64_t* strides,
+                        int32_t tokens, int32_t heads, int32_t head_dim, int32_t block_size,
+                        int32_t samples, float scale, float* mass, void* workspace,
+                        size_t workspace_bytes, hipStream_t stream);
+size_t dsa_sampled_mass_workspace_bytes(int32_t tokens, int32_t heads, int32_t block_size,
+                                        int32_t samples);
+
+/*
  * Exact block attention mass of one batch-1 self-attention call, bf16 or fp16
  * Q/K (dtype).
  * Replaces `_block_attention_mass` and its Triton `_exact_block_mass_kernel`

@@ -85,6 +85,86 @@ def test_sampled_mass_few_sampled_keys(ops, cuda_device, tokens, samples):
     np.testing.assert_allclose(got.sum(-1), 1.0, atol=1e-5)
 
 
+def _two_sweep_mass(q, k, block, samples):
+    """dsa_sampled_mass without a workspace: scores computed twice."""
+    from dit_sparse_atten_amd import _lib
+    _, tokens, heads, dim = q.shape
+    blocks = math.ceil(tokens / block)
+    mass = torch.empty((heads, blocks, blocks), dtype=torch.float32, device=q.device)
+    strides = _lib.int64_array([q.stride(1), q.stride(2), k.stride(1), k.stride(2)])
+    status = _lib.load().dsa_sampled_mass(
+        q.data_ptr(), k.data_ptr(), 0 if q.dtype == torch.bfloat16 else 1, strides, tokens,
+        heads, dim, block, samples, dim ** -0.5, mass.data_ptr(),
+        torch.cuda.current_stream().cuda_stream)
+    _lib.check(status, "dsa_sampled_mass")
+    return mass
+
+
+@pytest.mark.parametrize("tokens,block,samples,dim,growth", [
+    (130, 128, 16, 128, 1), (2049, 128, 8, 64, 1), (1500, 128, 16, 256, 1),
+    (3000, 128, 2, 128, 40), (3000, 64, 4, 128, 40), (3000, 128, 16, 128, 40),
+    (3000, 128, 12, 128, 40), (1000, 32, 32, 128, 40)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_sampled_mass_one_sweep_equals_two(ops, cuda_device, tokens, block, samples, dim, growth,
+                                           dtype):
+    """The one-sweep scan against the two-sweep one on the same inputs: ragged
+    blocks, and scores that outgrow a row's first reference (`growth`: later
+    keys up to 40 times longer, hundreds of log2 units), which moves it.  Both
+    take exp2 of fp32 differences of log2 scores of up to 2^11: each is within
+    2^-13 ln 2 of the exact term, 2.5e-4 together with the row sum."""
+    q, k, _ = clustered_qkv(tokens, 3, dim, group=block, seed=tokens + samples, dtype=dtype)
+    ramp = torch.linspace(1, growth, tokens).view(1, -1, 1, 1)
+    q = q.to(cuda_device)
+    k = (k.float() * ramp).to(dtype).to(cuda_device)
+    got, want = ops.sampled_block_mass(q, k, block, samples), _two_sweep_mass(q, k, block, samples)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(got, want, rtol=2.5e-4, atol=1e-9)
+    flipped = k.flip(1)  # the largest scores first: later terms vanish
+    torch.testing.assert_close(ops.sampled_block_mass(q, flipped, block, samples),
+                               _two_sweep_mass(q, flipped, block, samples), rtol=2.5e-4, atol=1e-9)
+
+
+def test_sampled_mass_one_sweep_non_finite_rows(ops, cuda_device):
+    """fp16 scores that overflow to +inf or -inf, and a NaN query: the same
+    rows are NaN as in the two-sweep scan, the others agree."""
+    q, k, _ = clustered_qkv(1024, 2, 128, group=128, seed=5, dtype=torch.float16)
+    q, k = q.to(cuda_device), k.to(cuda_device)
+    positions = [4 + 8 * s for s in range(16)]  # sampled tokens of a 128-token block
+    q[0, 256 + positions[3], 0] = float("nan")
+    q[0, 512 + positions[0]] = 60.0
+    k[0, 640 + positions[5]] = 60.0   # 460,800 against the row of 60s: +inf
+    k[0, 768 + positions[5]] = -60.0  # -inf
+    q[0, 128 + positions[1], 1] = -60.0
+    got, want = ops.sampled_block_mass(q, k, 128, 16), _two_sweep_mass(q, k, 128, 16)
+    torch.cuda.synchronize()
+    assert want.isnan().any() and not want.isnan().all()
+    torch.testing.assert_close(got, want, rtol=2.5e-4, atol=1e-9, equal_nan=True)
+
+
+def test_sampled_mass_one_sweep_in_several_launches(ops, cuda_device):
+    """1,040 workgroups over a workspace of 1,024 slots: two launches."""
+    from dit_sparse_atten_amd import _lib
+    lib = _lib.load()
+    tokens, heads, samples = 13312, 40, 32
+    generator = torch.Generator(device=cuda_device).manual_seed(2)
+    q, k = (torch.randn((1, tokens, heads, 128), device=cuda_device, generator=generator)
+            .to(torch.bfloat16) for _ in range(2))
+    full = lib.dsa_sampled_mass_workspace_bytes(tokens, heads, 128, samples)
+    groups = heads * 26
+    assert full % groups == 0
+    want = ops.sampled_block_mass(q, k, 128, samples)
+    workspace = torch.empty(full // groups * 1024, dtype=torch.uint8, device=cuda_device)
+    mass = torch.empty_like(want)
+    strides = _lib.int64_array([q.stride(1), q.stride(2), k.stride(1), k.stride(2)])
+    status = lib.dsa_sampled_mass_ws(
+        q.data_ptr(), k.data_ptr(), 0, strides, tokens, heads, 128, 128, samples, 128 ** -0.5,
+        mass.data_ptr(), workspace.data_ptr(), workspace.numel(),
+        torch.cuda.current_stream().cuda_stream)
+    _lib.check(status, "dsa_sampled_mass_ws")
+    torch.cuda.synchronize()
+    assert torch.equal(mass, want)
+
+
 def test_full_sampling_at_block_128_matches_exact_block_mass(ops, cuda_device):
     """samples == block == 128 (the reference's identity, test_flex_backend.py:
     43-53, at the production block size): mass = exact mass / block, up to
@@ -169,6 +249,24 @@ def test_route_select_prior_golden(ops, cuda_device):
     torch.cuda.synchronize()
     primed = R.persistence_prior(data["mass"], data["previous"], 0.5)
     assert (route.cpu().numpy() == R.top_mass_route(primed, 0.95, 0.625)).all()
+
+
+@pytest.mark.parametrize("keys", [1, 63, 64, 65, 128, 129, 256, 257])
+def test_route_select_short_rows(ops, cuda_device, keys):
+    """The 64-, 128- and 256-key instances at their edges, with the prior and a
+    sink, bit-exact; some values repeated."""
+    rng = np.random.default_rng(keys)
+    mass = rng.random((2, 9, keys)).astype(np.float32) ** 4
+    mass[:, :, ::5] = mass[:, :, :1]
+    previous = rng.random(mass.shape) < 0.5
+    route, counts = ops.route_select(
+        torch.from_numpy(mass).to(cuda_device), 0.9, 0.625,
+        previous=torch.from_numpy(previous).to(cuda_device), persistence=0.5, sink_blocks=2)
+    torch.cuda.synchronize()
+    expected = R.top_mass_route(R.persistence_prior(mass, previous, 0.5), 0.9, 0.625)
+    expected[..., :2] = True
+    assert (route.cpu().numpy() == expected).all()
+    assert (counts.cpu().numpy() == expected.sum(-1)).all()
 
 
 def test_route_select_rounding_boundaries(ops, cuda_device):
