@@ -90,6 +90,7 @@ int prepare(const void* q, const void* k, const void* v, void* o, int32_t dtype,
   p->drop_thresh = 0;
   p->drop_scale = 1.f;
   p->drop_seed_lo = p->drop_seed_hi = p->drop_offset = 0;
+  p->split_max = nullptr;
   p->scale = scale;
   p->scale_log2 = scale * 1.4426950408889634f;
   return DSA_OK;
@@ -99,8 +100,12 @@ int prepare(const void* q, const void* k, const void* v, void* o, int32_t dtype,
 // (launch order, then split partials; see launch_typed).
 int launch(int32_t dtype, BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t stream,
            const char* who) {
-  // fp32 inputs, dropout and head dims above 128 run the fp32-compute kernel
-  // (no scratch).
+  // fp32 inputs run as split fp16 products where the scratch holds them;
+  // without, dropout and head dims above 128 run the fp32-compute kernel (no
+  // scratch).
+  if (dtype == DSA_F32 && p.drop_thresh == 0 && p.head_dim <= kHeadDim &&
+      scratch_bytes >= split_workspace_bytes((int64_t)p.batch * p.heads, p.kv_tokens))
+    return bsa_launch_f32_split(p, scratch, stream, who);
   if (dtype == DSA_F32 || p.drop_thresh != 0 || p.head_dim > kHeadDim)
     return bsa_launch_f32(p, dtype, stream, who);
   return dtype == DSA_F16 ? bsa_launch_f16(p, scratch, scratch_bytes, stream, who)
@@ -320,6 +325,13 @@ extern "C" size_t dsa_bsa_workspace_bytes(int32_t batch, int32_t heads, int32_t 
   return dsa_bsa_workspace_bytes_block(batch, heads, kv_tokens, head_dim, 128);
 }
 
+extern "C" size_t dsa_bsa_f32_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
+                                              int32_t head_dim) {
+  if (batch <= 0 || heads <= 0 || kv_tokens <= 0 || head_dim <= 0 || head_dim > kHeadDim)
+    return 0;
+  return (split_workspace_bytes((int64_t)batch * heads, kv_tokens) + 255) & ~(size_t)255;
+}
+
 extern "C" int dsa_bsa_fwd(const void* q, const void* k, const void* v, void* o,
                            int32_t dtype, const int64_t* strides, int32_t batch, int32_t q_tokens,
                            int32_t kv_tokens, int32_t heads, int32_t head_dim,
@@ -360,7 +372,9 @@ extern "C" int dsa_bsa_fwd_noalloc(const void* q, const void* k, const void* v, 
   // Calls of more work items than the order region holds run in launch
   // order, as dsa_bsa_fwd does; the split never takes more partials than the
   // array holds.  So no call size needs more scratch than this.
-  return launch(dtype, p, area, kScratchBytes, stream, "dsa_bsa_fwd_noalloc");
+  // fp32 calls keep to the kernel that takes none, so they may overlap.
+  return launch(dtype, p, area, dtype == DSA_F32 ? 0 : kScratchBytes, stream,
+                "dsa_bsa_fwd_noalloc");
 }
 
 extern "C" int dsa_bsa_fwd_dropout(const void* q, const void* k, const void* v, void* o,

@@ -108,6 +108,9 @@ struct BsaParams {
   uint32_t drop_thresh;
   float drop_scale;
   uint32_t drop_seed_lo, drop_seed_hi, drop_offset;
+  // The fp32-compute kernel after bsa_fwd_split_kernel: its magnitude maxima
+  // (null: every head is this kernel's).
+  const uint32_t* split_max;
 };
 
 // One split partial: O [128 rows][128 dims] relative to the row's reference
@@ -1382,3 +1385,9 @@ int bsa_launch_f16(bsa::BsaParams p, void* scratch, size_t scratch_bytes, hipStr
 // fp32-compute kernel (bsa_fwd_f32.hip): fp32 inputs (dtype DSA_F32), dense
 // calls with dropout, and head dims 136..256, of any input type.
 int bsa_launch_f32(bsa::BsaParams p, int32_t dtype, hipStream_t stream, const char* who);
+// Split fp16 products (bsa_fwd_f32s.hip): fp32 inputs, head dims up to 128, no
+// dropout, on split_workspace_bytes of workspace.
+int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, hipStream_t stream, const char* who);
+namespace bsa {
+size_t split_workspace_bytes(int64_t pairs, int64_t kv_tokens);
+}

@@ -26,6 +26,7 @@ SOURCES = (
     "bsa_fwd.hip",
     "bsa_fwd_f16.hip",
     "bsa_fwd_f32.hip",
+    "bsa_fwd_f32s.hip",
     "block_mass.hip",
     "tile_stats.hip",
     "sampled_mass.hip",

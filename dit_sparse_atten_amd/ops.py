@@ -60,6 +60,14 @@ def _kernel_view(name, tensor, dtype=None, attention=False):
     return tensor if ok else tensor.contiguous()
 
 
+def _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim):
+    """Workspace of the float32 attention's split products (0 for the 16-bit
+    types and for head dims above 128)."""
+    if q.dtype != torch.float32:
+        return 0
+    return lib.dsa_bsa_f32_workspace_bytes(batch, heads, kv_tokens, head_dim)
+
+
 class RouteCSR:
     """Compressed block route: for every (route batch, head, query block) row,
     the ascending list of key blocks it attends to.
@@ -204,12 +212,14 @@ def bsa_fwd(q, k, v, csr=None, scale=None, out=None, return_lse=False, block_siz
         raise ValueError(f"block_size {block_size} unsupported (1..128)")
     deterministic = bool(deterministic) or torch.are_deterministic_algorithms_enabled()
     # Room for the split partials of the last round of workgroups (none when
-    # the key range is too short to split; the fp32-compute kernel, which
-    # also takes head dims above 128, uses none); the caching allocator
-    # recycles it.
-    fp32_kernel = q.dtype == torch.float32 or head_dim > HEAD_DIM
-    workspace_bytes = 0 if fp32_kernel else lib.dsa_bsa_workspace_bytes_block(
-        batch, heads, kv_tokens, head_dim, block_size)
+    # the key range is too short to split), or, in fp32, for the split K and V
+    # (head dims above 128 run the fp32-compute kernel, which uses none); the
+    # caching allocator recycles it.
+    if q.dtype == torch.float32 or head_dim > HEAD_DIM:
+        workspace_bytes = _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim)
+    else:
+        workspace_bytes = lib.dsa_bsa_workspace_bytes_block(
+            batch, heads, kv_tokens, head_dim, block_size)
     workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device)
                  if workspace_bytes else None)
     with torch.cuda.device(q.device):
@@ -339,6 +349,7 @@ def bsa_fwd_block_mass(q, k, v, scale=None):
         list(q.stride()[:3]) + list(k.stride()[:3]) + list(v.stride()[:3])
         + list(out.stride()[:3]))
     workspace_bytes = lib.dsa_bsa_fwd_block_mass_workspace_bytes(heads, tokens, head_dim)
+    workspace_bytes += _f32_workspace_bytes(lib, q, 1, heads, tokens, head_dim)
     workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device)
                  if workspace_bytes else None)
     with torch.cuda.device(q.device):
@@ -465,6 +476,7 @@ def bsa_fwd_tile_stats(q, k, v, csr, tile_shape, scale=None, deterministic=False
         + list(out.stride()[:3]))
     workspace_bytes = lib.dsa_bsa_fwd_tile_stats_workspace_bytes(
         heads, tokens, head_dim, tile_h, tile_w, entries)
+    workspace_bytes += _f32_workspace_bytes(lib, q, 1, heads, tokens, head_dim)
     workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device)
                  if workspace_bytes else None)
     with torch.cuda.device(q.device):

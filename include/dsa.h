@@ -121,6 +121,15 @@ int dsa_bsa_fwd(const void* q, const void* k, const void* v, void* o, int32_t dt
 size_t dsa_bsa_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
                                int32_t head_dim);
 
+/* Workspace bytes with which an fp32 call of head dim up to 128 (dsa_bsa_fwd;
+ * dsa_bsa_fwd_tile_stats and dsa_bsa_fwd_block_mass: beyond their own) runs
+ * every fp32 product as three fp16 products on the 16-bit matrix cores, at no
+ * larger error (a head with non-finite or extreme elements keeps the fp32
+ * products): the split K and V, 1,024 bytes per token, batch item and head.
+ * 0 above head dim 128.  With less workspace the fp32 kernel runs. */
+size_t dsa_bsa_f32_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
+                                   int32_t head_dim);
+
 /* The same for any block_size in 1..128 (key blocks of block_size tokens). */
 size_t dsa_bsa_workspace_bytes_block(int32_t batch, int32_t heads, int32_t kv_tokens,
                                      int32_t head_dim, int32_t block_size);

@@ -86,6 +86,69 @@ def test_fp32_routed_matches_float64(ops, cuda_device, tokens, block):
     assert (out[0, :block, 0] == 0).all()
 
 
+@pytest.mark.parametrize("tokens,heads,block,routed", [
+    (33, 8, 128, False), (130, 8, 64, True), (4096, 16, 64, True), (1100, 8, 100, True)])
+def test_fp32_split_heads_against_fp32_products(ops, cuda_device, monkeypatch, tokens, heads,
+                                                block, routed):
+    """Heads of very different magnitudes in one call, with the workspace (split
+    fp16 products) and without (fp32 products): each head by its own scales, and
+    heads with non-finite or extreme elements on the fp32 kernel, bit for bit.
+    2-wave workgroups with one stage (1,024 of them) and with two, 4-wave ones,
+    sub-tiles of 1, 2, 4 and 32 keys."""
+    q, k, v = (x.to(cuda_device) for x in _qkv(1, tokens, tokens, heads, 128, seed=tokens))
+    q[:, :, 1] *= 2.0 ** 20
+    k[:, :, 1] *= 2.0 ** -20
+    v[:, :, 1] *= 2.0 ** -30
+    v[:, :, 2] *= 2.0 ** 30
+    q[:, :, 2] = 0
+    q[:, :, 3] *= 1e-30              # extreme: fp32 products
+    v[0, tokens // 2, 4, 5] = float("inf")
+    k[0, tokens - 1, 5, 0] = float("nan")
+    q[0, 0, 6, 0] = float("-inf")
+    k[0, 3, 7] *= 2.0 ** 20          # one token far above the others
+    csr = None
+    if routed:
+        blocks = math.ceil(tokens / block)
+        route = random_route(heads, blocks, seed=block, keep=0.5)
+        csr = ops.route_to_csr(route.to(cuda_device), block_size=block)
+    got, got_lse = ops.bsa_fwd(q, k, v, csr, return_lse=True, block_size=block)
+    monkeypatch.setattr(ops, "_f32_workspace_bytes", lambda *args: 0)
+    want, want_lse = ops.bsa_fwd(q, k, v, csr, return_lse=True, block_size=block)
+    torch.cuda.synchronize()
+    for head, scale in enumerate((1.0, 2.0 ** -30, 2.0 ** 30)):
+        # Two fp32 results, each within OUT_ATOL of float64 at |v| of order one.
+        torch.testing.assert_close(got[:, :, head] / scale, want[:, :, head] / scale,
+                                   atol=2 * OUT_ATOL, rtol=0)
+        torch.testing.assert_close(got_lse[:, head], want_lse[:, head], atol=2 * LSE_ATOL, rtol=0)
+    assert not torch.equal(got[:, :, 0], want[:, :, 0])  # two different kernels ran
+    for head in range(3, 8):
+        assert torch.equal(got[:, :, head].view(torch.int32), want[:, :, head].view(torch.int32))
+        assert torch.equal(got_lse[:, head].view(torch.int32),
+                           want_lse[:, head].view(torch.int32))
+
+
+@pytest.mark.parametrize("tokens,routed", [(1024, False), (6000, False), (6016, True)])
+def test_fp32_split_error_is_no_larger(ops, cuda_device, monkeypatch, tokens, routed):
+    """Relative error of O against float64 (torch, on the device): the split
+    products' is at most that of the fp32 products."""
+    q, k, v = (x.to(cuda_device) for x in _qkv(1, tokens, tokens, 2, 128, seed=tokens))
+    route = torch.ones(2, -(-tokens // 128), -(-tokens // 128), dtype=torch.bool)
+    if routed:
+        route = random_route(2, route.shape[1], seed=3, keep=0.5)
+    csr = ops.route_to_csr(route.to(cuda_device)) if routed else None
+    keep = route.to(cuda_device).repeat_interleave(128, 1).repeat_interleave(128, 2)
+    s = (q[0].double().transpose(0, 1) @ k[0].double().permute(1, 2, 0).contiguous()) * 128 ** -0.5
+    s.masked_fill_(~keep[:, :tokens, :tokens], -math.inf)
+    exact = (torch.softmax(s, dim=-1) @ v[0].double().transpose(0, 1).contiguous()).transpose(0, 1)
+    errors = []
+    for workspace in (True, False):
+        if not workspace:
+            monkeypatch.setattr(ops, "_f32_workspace_bytes", lambda *args: 0)
+        out = ops.bsa_fwd(q, k, v, csr)[0].double()
+        errors.append(((out - exact).norm() / exact.norm()).item())
+    assert errors[0] <= errors[1] <= 1e-5, errors
+
+
 def _tile_inputs(grid, tile, heads, seed):
     case = S.SparsePathCase(grid, tile=tile)
     tokens = grid[0] * grid[1] * grid[2]
