@@ -37,7 +37,7 @@
 //    the final row sum pair lanes l and l ^ 32 with v_permlane32_swap;
 //  * query / key blocks of 1..128 tokens (the matrix-sparse backend's spatial
 //    tiles): routed whole blocks of 65..127 keys stream the row's kept blocks
-//    as one gathered key sequence (kGather), and routed blocks of at most 64
+//    as one gathered key sequence (up to 96 in bsa_narrow.h, above kGather), and routed blocks of at most 64
 //    tokens run 2-wave workgroups (kWaves);
 //  * the last, partial round of query blocks may run as 2..8 key ranges each
 //    (choose_split), whose fp32 partials bsa_merge_kernel combines;
@@ -1025,6 +1025,10 @@ __global__ void __launch_bounds__(kWaves * 64, 2)
   }
 }
 
+}  // namespace bsa
+#include "bsa_narrow.h"
+namespace bsa {
+
 // Launch order of a routed call: within each (batch, head) group its query
 // blocks by key-block count descending, ties by index ascending (a stable
 // sort), so the workgroups that run side by side walk rows of similar length
@@ -1293,10 +1297,18 @@ int launch_typed(BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t s
   // Blocks whose last half-tile holds 1..32 keys run it as one sub-tile.
   const int rem = p.block % kHalfKeys;
   const bool skip = rem != 0 && rem <= 32;
-  const bool gather = p.row_ptr && use_gather(p.block, p.kv_tokens, p.k_st, p.v_st);
-  // Resident workgroups: two per CU, four for the single-stage 2-wave ones
-  // (routed blocks, or dense statistics, of at most 64 keys).
-  const bool two_wave = nh == 1 && (p.row_ptr || p.rs_logm);
+  // Routed whole blocks of 65..96 tokens: 16-row groups (bsa_narrow.h) where the
+  // call fills a CU's four 2-wave workgroups; with fewer, three waves to a tile
+  // finish it sooner (72-token tiles, the 32-row gathered stream against
+  // bsa_narrow.h: 768 tiles with statistics 238 / 256 us, 192 tiles 86 / 95; 1,056
+  // tiles 384 / 363, 1,200 tiles 457 / 423, 8,000 tiles 4.78 / 4.30 ms).  The
+  // gathered stream also takes blocks of 97..127.
+  const bool narrow = p.row_ptr && grid > 2 * device_slots(stream) &&
+                      use_narrow(p.block, p.kv_tokens, p.k_st, p.v_st);
+  const bool gather = narrow || (p.row_ptr && use_gather(p.block, p.kv_tokens, p.k_st, p.v_st));
+  // Resident workgroups: two per CU, four for the 2-wave ones (routed blocks,
+  // or dense statistics, of at most 64 keys; narrow).
+  const bool two_wave = narrow || (nh == 1 && (p.row_ptr || p.rs_logm));
   const int slots = device_slots(stream) * (two_wave ? 2 : 1);
   if (lead > 0 && scratch_bytes >= lead) {
     unsigned char* base = static_cast<unsigned char*>(scratch);
@@ -1345,7 +1357,10 @@ int launch_typed(BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t s
       two_waves(128);
   auto four = [&](auto kernel) { hipLaunchKernelGGL(kernel, blocks, threads, 0, stream, p); };
   auto two = [&](auto kernel) { hipLaunchKernelGGL(kernel, blocks, two_waves, 0, stream, p); };
-  if (gather) {
+  if (narrow) {
+    if (p.rs_logm) two(bsa_fwd_narrow_kernel<T, true>);
+    else two(bsa_fwd_narrow_kernel<T, false>);
+  } else if (gather) {
     if (p.rs_logm) four(bsa_fwd_kernel<T, true, 2, true, true, 4, true>);
     else four(bsa_fwd_kernel<T, true, 2, true, true>);
   } else if (p.row_ptr && p.rs_logm) {

@@ -37,7 +37,7 @@ typedef short dsa_i16x4 __attribute__((ext_vector_type(4)));
 
 namespace dsa {
 
-// The 16-bit input types share one MFMA shape (32x32x16, fp32 accumulate)
+// The 16-bit input types share their MFMA shapes (fp32 accumulate)
 // and one LDS layout; Elem<T> names the vector types and the matrix op.
 template <typename T>
 struct Elem;
@@ -50,6 +50,9 @@ struct Elem<__bf16> {
   static __device__ __forceinline__ dsa_f32x16 mfma32(x8 a, x8 b, dsa_f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ dsa_f32x4 mfma16(x8 a, x8 b, dsa_f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
 };
 
 template <>
@@ -59,6 +62,9 @@ struct Elem<_Float16> {
   typedef dsa_f16x2 x2;
   static __device__ __forceinline__ dsa_f32x16 mfma32(x8 a, x8 b, dsa_f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ dsa_f32x4 mfma16(x8 a, x8 b, dsa_f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
 };
 

@@ -441,6 +441,50 @@ def test_key_norm_bound_gathered_stream(cuda_device, block):
     _check(out, q, k, v, route, block=block)
 
 
+@pytest.mark.parametrize("block,blocks,heads,head_dim", [
+    (65, 9, 115, 128), (72, 20, 52, 72), (80, 9, 115, 8), (81, 9, 115, 128), (96, 9, 115, 120),
+    (72, 32, 34, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_narrow_blocks(cuda_device, block, blocks, heads, head_dim, dtype):
+    """Routed 65..96-token blocks in more than 1,024 workgroups (16-row groups: 5
+    of them up to 80 rows, then 6): NaN in the storage beside every row's head_dim elements, an empty row,
+    one-block rows, keys that grow along the sequence (references that move),
+    a split last round (1,088 workgroups of 32 key blocks); with a workspace and without (no
+    key norms: every chunk takes its row max)."""
+    from dit_sparse_atten_amd import _lib
+    from dit_sparse_atten_amd.ops import bsa_fwd, csr_from_route
+    tokens = block * blocks
+    generator = torch.Generator().manual_seed(block + head_dim)
+    storage = torch.full((3, 1, tokens, heads, 128), float("nan"))
+    storage[..., :head_dim] = torch.randn((3, 1, tokens, heads, head_dim), generator=generator)
+    storage[1, ..., :head_dim] *= torch.linspace(0.2, 3.0, tokens).view(1, -1, 1, 1)
+    storage = storage.to(dtype)
+    q, k, v = storage[..., :head_dim]
+    route = torch.rand(1, heads, blocks, blocks, generator=generator) < 0.6
+    route[0, 0, 1] = False
+    route[0, 1, 2] = False
+    route[0, 1, 2, blocks - 1] = True
+    qd, kd, vd = storage.to(cuda_device)[..., :head_dim]
+    csr = csr_from_route(route.to(cuda_device), block_size=block)
+    out, lse = bsa_fwd(qd, kd, vd, csr, block_size=block, return_lse=True)
+    bare = torch.empty_like(out)
+    strides = _lib.int64_array([s for t in (qd, kd, vd, bare) for s in t.stride()[:3]])
+    status = _lib.load().dsa_bsa_fwd(
+        qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), bare.data_ptr(),
+        0 if dtype == torch.bfloat16 else 1, strides, 1, tokens, tokens, heads, head_dim, block,
+        csr.row_ptr.data_ptr(), csr.col_idx.data_ptr(), 1, head_dim ** -0.5, 0, 0, None, None, 0,
+        torch.cuda.current_stream().cuda_stream)
+    _lib.check(status, "dsa_bsa_fwd")
+    torch.cuda.synchronize()
+    _check(out, q, k, v, route, block=block)
+    _check(bare, q, k, v, route, block=block)
+    assert (out[0, block:2 * block, 0] == 0).all()
+    _, want = block_sparse_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(),
+                                     route.numpy(), block)
+    # fp32 sums of exactly representable products; -inf for the empty row.
+    np.testing.assert_allclose(lse.cpu().numpy(), want, atol=1e-4, rtol=0)
+
+
 @pytest.mark.parametrize("routed", [False, True])
 def test_key_norm_bound_fp16_late_large_scores(cuda_device, routed):
     """fp16 P overflows above 65,504: a row whose walk starts on keys it barely
