@@ -91,6 +91,14 @@ int prepare(const void* q, const void* k, const void* v, void* o, int32_t dtype,
   p->drop_scale = 1.f;
   p->drop_seed_lo = p->drop_seed_hi = p->drop_offset = 0;
   p->split_max = nullptr;
+  // Set by the launchers that use them.
+  p->order = nullptr;
+  p->queue = nullptr;
+  p->walk = nullptr;
+  p->kv_norm = nullptr;
+  p->part = nullptr;
+  p->parts = 1;
+  p->split_from = (int32_t)grid;
   p->scale = scale;
   p->scale_log2 = scale * 1.4426950408889634f;
   return DSA_OK;
@@ -105,7 +113,7 @@ int launch(int32_t dtype, BsaParams p, void* scratch, size_t scratch_bytes, hipS
   // scratch).
   if (dtype == DSA_F32 && p.drop_thresh == 0 && p.head_dim <= kHeadDim &&
       scratch_bytes >= split_workspace_bytes((int64_t)p.batch * p.heads, p.kv_tokens))
-    return bsa_launch_f32_split(p, scratch, stream, who);
+    return bsa_launch_f32_split(p, scratch, scratch_bytes, stream, who);
   if (dtype == DSA_F32 || p.drop_thresh != 0 || p.head_dim > kHeadDim)
     return bsa_launch_f32(p, dtype, stream, who);
   return dtype == DSA_F16 ? bsa_launch_f16(p, scratch, scratch_bytes, stream, who)
@@ -329,7 +337,8 @@ extern "C" size_t dsa_bsa_f32_workspace_bytes(int32_t batch, int32_t heads, int3
                                               int32_t head_dim) {
   if (batch <= 0 || heads <= 0 || kv_tokens <= 0 || head_dim <= 0 || head_dim > kHeadDim)
     return 0;
-  return (split_workspace_bytes((int64_t)batch * heads, kv_tokens) + 255) & ~(size_t)255;
+  return split_workspace_bytes((int64_t)batch * heads, kv_tokens) +
+         (size_t)kMaxPartGroups * kPartBytes;
 }
 
 extern "C" int dsa_bsa_fwd(const void* q, const void* k, const void* v, void* o,

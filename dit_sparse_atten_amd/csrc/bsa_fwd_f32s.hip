@@ -141,8 +141,17 @@ __global__ void __launch_bounds__(kWaves * 64, 2) bsa_fwd_split_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5;
   const int qi = lane & 31;
-  const int work =
-      kRouted ? (int)blockIdx.x : dsa::xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  // Split last round, as in bsa_fwd_kernel (bsa_merge_kernel combines the parts).
+  const int wg = (int)blockIdx.x;
+  const bool split = wg >= p.split_from;
+  int work = wg, part = 0;
+  if (split) {
+    const int t = wg - p.split_from;
+    work = p.split_from + t / p.parts;
+    part = t % p.parts;
+  } else if (!kRouted) {
+    work = dsa::xcd_remap(wg, p.split_from);
+  }
   const int qb = work % p.q_blocks;
   const int bh = work / p.q_blocks;
   const int h = bh % p.heads;
@@ -162,6 +171,11 @@ __global__ void __launch_bounds__(kWaves * 64, 2) bsa_fwd_split_kernel(
     const int64_t row = ((int64_t)rb * p.heads + h) * p.q_blocks + qb;
     start = rp[row];
     end = rp[row + 1];
+  }
+  if (split) {
+    const int n = end - start;
+    end = start + (int)((int64_t)n * (part + 1) / p.parts);
+    start = start + (int)((int64_t)n * part / p.parts);
   }
   const dsa_const_i32 cidx = (dsa_const_i32)p.col_idx;
   const int nblk = end - start;
@@ -418,6 +432,24 @@ __global__ void __launch_bounds__(kWaves * 64, 2) bsa_fwd_split_kernel(
   }
 
   const float l_tot = dsa::pair32_sum(l_run);
+  if (split) {
+    if (row_ok) {
+      float* po = p.part + (int64_t)(wg - p.split_from) * kPartFloats;
+      const float unscale = sc.out * kPUnscale;  // powers of two
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr)
+          *reinterpret_cast<dsa_f32x4*>(po + local_row * kHeadDim + dt * 32 + rr * 8 + g * 4) =
+              dsa_f32x4{oacc[dt][rr * 4 + 0] * unscale, oacc[dt][rr * 4 + 1] * unscale,
+                        oacc[dt][rr * 4 + 2] * unscale, oacc[dt][rr * 4 + 3] * unscale};
+      if (g == 0) {
+        po[128 * 128 + local_row] = m_run;
+        po[128 * 128 + 128 + local_row] = l_tot * kPUnscale;
+      }
+    }
+    return;
+  }
   const float inv = (l_tot > 0.f ? 1.f / l_tot : 0.f) * sc.out;
   if (row_ok) {
     float* orow = static_cast<float*>(p.o) + b * p.o_sb + h * p.o_sh + (int64_t)tq * p.o_st;
@@ -438,19 +470,19 @@ __global__ void __launch_bounds__(kWaves * 64, 2) bsa_fwd_split_kernel(
 }
 
 // Bytes of the magnitude maxima and the split K and V of `pairs` (batch, head)
-// pairs.
+// pairs, rounded up to 256.
 size_t split_workspace_bytes(int64_t pairs, int64_t kv_tokens) {
-  return (size_t)(3 * pairs * kMaxParts * (int64_t)sizeof(uint32_t) +
-                  2 * pairs * kv_tokens * kSplitRow);
+  return round256((size_t)(3 * pairs * kMaxParts * (int64_t)sizeof(uint32_t) +
+                           2 * pairs * kv_tokens * kSplitRow));
 }
 
 }  // namespace bsa
 
-// Launches a prepared float32 call (head dim up to 128, no dropout) on
-// split_workspace_bytes of 16-byte aligned workspace: the heads that run here,
-// then the fp32 kernel over the rest.
-int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, hipStream_t stream,
-                         const char* who) {
+// Launches a prepared float32 call (head dim up to 128, no dropout) on at least
+// split_workspace_bytes of 16-byte aligned workspace (what follows them holds
+// split partials): the heads that run here, then the fp32 kernel over the rest.
+int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, size_t workspace_bytes,
+                         hipStream_t stream, const char* who) {
   using namespace bsa;
   const unsigned pairs = (unsigned)(p.batch * p.heads);
   uint32_t* parts = static_cast<uint32_t*>(workspace);
@@ -461,13 +493,25 @@ int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, hipStream_t stream,
                      dim3((unsigned)((p.kv_tokens + kSplitTokens - 1) / kSplitTokens), pairs, 2),
                      dim3(256), 0, stream, p, parts, planes);
   const int64_t grid = (int64_t)pairs * p.q_blocks;
-  const dim3 blocks((unsigned)grid);
+  // 2-wave workgroups with two stages put two on a CU, with one stage four:
+  // the latter where the call has more than two per CU.
+  const int slots = device_slots(stream);
+  const bool two = p.block <= 64, single = grid > slots;
+  // Split last round: a 4-wave workgroup alone on a CU runs nearly twice as fast
+  // as one of two, so a round is one per CU (2-wave ones: two).  3,600 tokens x
+  // 12 heads (348 workgroups, 92 in five parts) 288 -> 242 us; a part keeps at
+  // least four key blocks.
+  const size_t lead = split_workspace_bytes(pairs, p.kv_tokens);
+  p.part = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + lead);
+  p.parts = 1;
+  const int split = choose_split(
+      grid, two ? slots : slots / 2, std::min(8, p.kv_blocks / 4),
+      std::min<int64_t>((int64_t)((workspace_bytes - lead) / kPartBytes), kMaxPartGroups), &p.parts);
+  p.split_from = (int32_t)(grid - split);
+  const dim3 blocks((unsigned)(grid - split + (int64_t)split * p.parts));
   auto run = [&](auto kernel, int waves) {
     hipLaunchKernelGGL(kernel, blocks, dim3((unsigned)waves * 64), 0, stream, p, parts, planes);
   };
-  // 2-wave workgroups with two stages put two on a CU, with one stage four:
-  // the latter where the call has more than two per CU.
-  const bool two = p.block <= 64, single = grid > device_slots(stream);
   if (p.row_ptr) {
     if (p.rs_logm) {
       if (!two) run(bsa_fwd_split_kernel<true, true, 4, false>, 4);
@@ -489,6 +533,7 @@ int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, hipStream_t stream,
       else run(bsa_fwd_split_kernel<false, false, 2, false>, 2);
     }
   }
+  if (split > 0) launch_merge<float>(p, split, stream);
   p.split_max = parts;
   return bsa_launch_f32(p, DSA_F32, stream, who);
 }

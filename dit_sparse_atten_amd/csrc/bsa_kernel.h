@@ -1141,57 +1141,91 @@ __global__ void __launch_bounds__(256) key_norm_kernel(BsaParams p, float* out) 
 
 // Combines the `parts` partials of each split query block: with M the largest
 // row max, O = sum_i O_i 2^(m_i - M) / sum_i l_i 2^(m_i - M) and
-// LSE = M ln 2 + ln(sum_i l_i 2^(m_i - M)).  Two threads per row, 64 dims each.
+// LSE = M ln 2 + ln(sum_i l_i 2^(m_i - M)).  Latency-bound (66 KB per part over
+// a few dozen to 500 query blocks): a workgroup takes kMergeRows rows of one
+// block, eight threads to a row with 16 dims each, and every thread has four
+// parts' loads on their way at once.  One workgroup per block with two threads
+// to a row took 16 us for 136 blocks of three parts; this takes 7.8.
+constexpr int kMergeRows = 32;
 template <typename T>
 __global__ void __launch_bounds__(256) bsa_merge_kernel(BsaParams p) {
-  const int item = blockIdx.x;
+  const int item = blockIdx.x / (128 / kMergeRows);
   const int work = p.order ? p.order[p.split_from + item] : p.split_from + item;
   const int qb = work % p.q_blocks;
   const int bh = work / p.q_blocks;
   const int h = bh % p.heads;
   const int b = bh / p.heads;
-  const int r = threadIdx.x >> 1, half = threadIdx.x & 1;
+  const int r = (blockIdx.x % (128 / kMergeRows)) * kMergeRows + (threadIdx.x >> 3);
+  const int d0 = (threadIdx.x & 7) * 16;
   const int tq = qb * p.block + r;
   if (r >= p.block || tq >= p.q_tokens) return;
   const float* base = p.part + (int64_t)item * p.parts * kPartFloats;
+  // Parts past the last repeat it, with weight 0.
+  float m[8], w[8];
   float m_max = -INFINITY;
-  for (int i = 0; i < p.parts; ++i) m_max = fmaxf(m_max, base[i * kPartFloats + 128 * 128 + r]);
-  float w[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float* part = base + (int64_t)min(i, p.parts - 1) * kPartFloats + 128 * 128 + r;
+    m[i] = part[0];
+    w[i] = part[128];
+    m_max = fmaxf(m_max, m[i]);
+  }
   float l = 0.f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    w[i] = 0.f;
-    if (i < p.parts) {
-      const float m_i = base[i * kPartFloats + 128 * 128 + r];
-      w[i] = m_i == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_i - m_max);
-      l = fmaf(w[i], base[i * kPartFloats + 128 * 128 + 128 + r], l);
-    }
+    const float l_i = w[i];
+    w[i] = i >= p.parts || m[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[i] - m_max);
+    if (i < p.parts) l = fmaf(w[i], l_i, l);
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  T* orow = static_cast<T*>(p.o) + b * p.o_sb + h * p.o_sh + (int64_t)tq * p.o_st;
-  for (int c = half * 8; c < half * 8 + 8; ++c) {  // 8-dim chunks of this thread's 64
-    if (c * 8 >= p.head_dim) break;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (i >= p.parts) break;
-      const float* src = base + i * kPartFloats + r * kHeadDim + c * 8;
-      const dsa_f32x4 a = *reinterpret_cast<const dsa_f32x4*>(src);
-      const dsa_f32x4 bq = *reinterpret_cast<const dsa_f32x4*>(src + 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[e] = fmaf(w[i], a[e], acc[e]);
-        acc[4 + e] = fmaf(w[i], bq[e], acc[4 + e]);
-      }
-    }
-    typename dsa::Elem<T>::x8 out;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) out[e] = (T)(acc[e] * inv);
-    *reinterpret_cast<typename dsa::Elem<T>::x8*>(orow + c * 8) = out;
-  }
-  if (p.lse && half == 0)
+  if (p.lse && d0 == 0)
     p.lse[((int64_t)b * p.heads + h) * p.q_tokens + tq] =
         l > 0.f ? m_max * 0.6931471805599453f + logf(l) : -INFINITY;
+  if (d0 >= p.head_dim) return;
+  float acc[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int i0 = 0; i0 < 8; i0 += 4) {
+    if (i0 >= p.parts) break;
+    dsa_f32x4 x[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        x[u][c] = *reinterpret_cast<const dsa_f32x4*>(
+            base + (int64_t)min(i0 + u, p.parts - 1) * kPartFloats + r * kHeadDim + d0 + 4 * c);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (i0 + u >= p.parts) break;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[e] = fmaf(w[i0 + u], x[u][e >> 2][e & 3], acc[e]);
+    }
+  }
+  T* orow = static_cast<T*>(p.o) + b * p.o_sb + h * p.o_sh + (int64_t)tq * p.o_st + d0;
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {  // rows are 16-byte aligned
+    if (d0 + c * 8 >= p.head_dim) break;
+    if constexpr (sizeof(T) == 4) {
+      dsa_f32x4* const dst = reinterpret_cast<dsa_f32x4*>(orow + c * 8);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        dst[u] = dsa_f32x4{acc[8 * c + 4 * u] * inv, acc[8 * c + 4 * u + 1] * inv,
+                           acc[8 * c + 4 * u + 2] * inv, acc[8 * c + 4 * u + 3] * inv};
+    } else {
+      typename dsa::Elem<T>::x8 out;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) out[e] = (T)(acc[8 * c + e] * inv);
+      *reinterpret_cast<typename dsa::Elem<T>::x8*>(orow + c * 8) = out;
+    }
+  }
+}
+
+// Launches it over the `split` split query blocks of a call.
+template <typename T>
+void launch_merge(const BsaParams& p, int split, hipStream_t stream) {
+  hipLaunchKernelGGL(bsa_merge_kernel<T>, dim3((unsigned)(split * (128 / kMergeRows))), dim3(256),
+                     0, stream, p);
 }
 
 inline bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
@@ -1287,10 +1321,6 @@ int launch_typed(BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t s
                  const char* who) {
   const int64_t grid = (int64_t)p.batch * p.heads * p.q_blocks;
   size_t used = 0;
-  p.order = nullptr;
-  p.walk = nullptr;
-  p.queue = nullptr;
-  p.kv_norm = nullptr;
   const int64_t norms = (int64_t)p.batch * p.heads;
   const size_t lead = order_bytes(grid, p.q_blocks, norms);
   const int32_t nh = p.block > kHalfKeys ? 2 : 1;
@@ -1387,8 +1417,7 @@ int launch_typed(BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t s
     if (nh == 2) skip ? four(bsa_fwd_kernel<T, false, 2, true>) : four(bsa_fwd_kernel<T, false, 2, false>);
     else skip ? four(bsa_fwd_kernel<T, false, 1, true>) : four(bsa_fwd_kernel<T, false, 1, false>);
   }
-  if (split > 0)
-    hipLaunchKernelGGL(bsa_merge_kernel<T>, dim3((unsigned)split), dim3(256), 0, stream, p);
+  if (split > 0) launch_merge<T>(p, split, stream);
   return dsa::check_launch(who);
 }
 
@@ -1401,8 +1430,9 @@ int bsa_launch_f16(bsa::BsaParams p, void* scratch, size_t scratch_bytes, hipStr
 // calls with dropout, and head dims 136..256, of any input type.
 int bsa_launch_f32(bsa::BsaParams p, int32_t dtype, hipStream_t stream, const char* who);
 // Split fp16 products (bsa_fwd_f32s.hip): fp32 inputs, head dims up to 128, no
-// dropout, on split_workspace_bytes of workspace.
-int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, hipStream_t stream, const char* who);
+// dropout, on at least split_workspace_bytes of workspace.
+int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, size_t workspace_bytes,
+                         hipStream_t stream, const char* who);
 namespace bsa {
 size_t split_workspace_bytes(int64_t pairs, int64_t kv_tokens);
 }

@@ -125,8 +125,10 @@ size_t dsa_bsa_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
  * dsa_bsa_fwd_tile_stats and dsa_bsa_fwd_block_mass: beyond their own) runs
  * every fp32 product as three fp16 products on the 16-bit matrix cores, at no
  * larger error (a head with non-finite or extreme elements keeps the fp32
- * products): the split K and V, 1,024 bytes per token, batch item and head.
- * 0 above head dim 128.  With less workspace the fp32 kernel runs. */
+ * products): the split K and V, 1,024 bytes per token, batch item and head, and
+ * 768 per batch item and head (rounded up to 256), then 68,157,440 for a split
+ * last round (optional).  0 above head dim 128.  With less workspace the fp32
+ * kernel runs. */
 size_t dsa_bsa_f32_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
                                    int32_t head_dim);
 

@@ -94,7 +94,8 @@ def test_fp32_split_heads_against_fp32_products(ops, cuda_device, monkeypatch, t
     fp16 products) and without (fp32 products): each head by its own scales, and
     heads with non-finite or extreme elements on the fp32 kernel, bit for bit.
     2-wave workgroups with one stage (1,024 of them) and with two, 4-wave ones,
-    sub-tiles of 1, 2, 4 and 32 keys."""
+    sub-tiles of 1, 2, 4 and 32 keys, and (1,100 tokens: 88 workgroups, 11 key
+    blocks) every query block in two key ranges."""
     q, k, v = (x.to(cuda_device) for x in _qkv(1, tokens, tokens, heads, 128, seed=tokens))
     q[:, :, 1] *= 2.0 ** 20
     k[:, :, 1] *= 2.0 ** -20
