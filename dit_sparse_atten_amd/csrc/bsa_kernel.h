@@ -1327,13 +1327,14 @@ int launch_typed(BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t s
   // Blocks whose last half-tile holds 1..32 keys run it as one sub-tile.
   const int rem = p.block % kHalfKeys;
   const bool skip = rem != 0 && rem <= 32;
-  // Routed whole blocks of 65..96 tokens: 16-row groups (bsa_narrow.h) where the
-  // call fills a CU's four 2-wave workgroups; with fewer, three waves to a tile
-  // finish it sooner (72-token tiles, the 32-row gathered stream against
-  // bsa_narrow.h: 768 tiles with statistics 238 / 256 us, 192 tiles 86 / 95; 1,056
-  // tiles 384 / 363, 1,200 tiles 457 / 423, 8,000 tiles 4.78 / 4.30 ms).  The
-  // gathered stream also takes blocks of 97..127.
-  const bool narrow = p.row_ptr && grid > 2 * device_slots(stream) &&
+  // Tile blocks of 65..96 tokens, routed or dense with statistics: 16-row groups
+  // (bsa_narrow.h) where the call fills a CU's four 2-wave workgroups; with
+  // fewer, three waves to a tile finish it sooner (72-token tiles, the 32-row
+  // gathered stream against bsa_narrow.h: 768 tiles with statistics 238 / 256 us,
+  // 192 tiles 86 / 95; 1,056 tiles 384 / 363, 1,200 tiles 457 / 423, 8,000 tiles
+  // 4.78 / 4.30 ms).  The gathered stream also takes blocks of 97..127.
+  const bool tiles = p.row_ptr || (p.rs_logm && p.stat_tile == p.block);
+  const bool narrow = tiles && grid > 2 * device_slots(stream) &&
                       use_narrow(p.block, p.kv_tokens, p.k_st, p.v_st);
   const bool gather = narrow || (p.row_ptr && use_gather(p.block, p.kv_tokens, p.k_st, p.v_st));
   // Resident workgroups: two per CU, four for the 2-wave ones (routed blocks,
@@ -1388,8 +1389,9 @@ int launch_typed(BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t s
   auto four = [&](auto kernel) { hipLaunchKernelGGL(kernel, blocks, threads, 0, stream, p); };
   auto two = [&](auto kernel) { hipLaunchKernelGGL(kernel, blocks, two_waves, 0, stream, p); };
   if (narrow) {
-    if (p.rs_logm) two(bsa_fwd_narrow_kernel<T, true>);
-    else two(bsa_fwd_narrow_kernel<T, false>);
+    if (!p.row_ptr) two(bsa_fwd_narrow_kernel<T, false, true>);
+    else if (p.rs_logm) two(bsa_fwd_narrow_kernel<T, true, true>);
+    else two(bsa_fwd_narrow_kernel<T, true, false>);
   } else if (gather) {
     if (p.rs_logm) four(bsa_fwd_kernel<T, true, 2, true, true, 4, true>);
     else four(bsa_fwd_kernel<T, true, 2, true, true>);

@@ -1,6 +1,7 @@
-// Routed attention on tile blocks of 65..96 tokens (gfx950), bf16 or fp16:
-// the gathered key stream of bsa_fwd_kernel with query rows in groups of 16.
-// Included by bsa_kernel.h, whose definitions it uses.
+// Attention on tile blocks of 65..96 tokens (gfx950), bf16 or fp16: the gathered
+// key stream of bsa_fwd_kernel with query rows in groups of 16.  Routed calls,
+// and dense ones (kRouted = false: every block listed) that take statistics of
+// such tiles.  Included by bsa_kernel.h, whose definitions it uses.
 //
 // On the 32-row MFMAs of bsa_fwd_kernel a 72-row query tile fills three waves'
 // 96 rows and leaves the fourth wave of a workgroup idle, so a CU's two
@@ -14,7 +15,9 @@
 // chunk from L2 for 72 rows (607 GB per call; without the loads, timing only,
 // 39 ms) and the wave that holds three of the five groups (two each: 42 ms).
 // Longer prefetch (32-key double-buffered stages) and three waves of two groups
-// measured no faster.
+// measured no faster; blocks of 57..64 tokens (two groups per wave) ran equal to
+// the 32-row 2-wave kernel.  Dense statistics, 240 tiles x 40 heads: 5 x 13
+// tokens 14.3 -> 9.4 ms, 9 x 10 tokens 15.0 -> 13.2 ms.
 //
 // Layouts (lane = 16 q4 + c16): S^T = K Q^T leaves lane (q4, c16) the keys
 // 16 kg + 4 q4 + r of query row c16 (r = 0..3), and two 16-key groups' values
@@ -41,7 +44,7 @@ constexpr int kNarrowWRows = 7;    // 2 parities x 3 kinds, then a zero row
 // read touches 16 key rows x 32 bytes, eight rows (256 bytes) at a time.
 __device__ __forceinline__ int v8_swz(int r, int c) { return c ^ (2 * (r & 7)); }
 
-template <typename T, bool kStats>
+template <typename T, bool kRouted, bool kStats>
 __global__ void __launch_bounds__(128, 2) bsa_fwd_narrow_kernel(BsaParams p) {
   typedef dsa::Elem<T> E;
   typedef typename E::x8 x8;
@@ -73,15 +76,19 @@ __global__ void __launch_bounds__(128, 2) bsa_fwd_narrow_kernel(BsaParams p) {
     part = t % p.parts;
   }
   int work = slot;
-  if (p.order) work = ((dsa_const_i32)p.order)[slot];
+  if (kRouted && p.order) work = ((dsa_const_i32)p.order)[slot];
   const int qb = work % p.q_blocks;
   const int bh = work / p.q_blocks;
   const int h = bh % p.heads;
   const int b = bh / p.heads;
-  const dsa_const_i32 rp = (dsa_const_i32)p.row_ptr;
-  const int rb = p.route_batches == 1 ? 0 : b;
-  const int64_t csr_row = ((int64_t)rb * p.heads + h) * p.q_blocks + qb;
-  int start = rp[csr_row], end = rp[csr_row + 1];
+  int start = 0, end = p.kv_blocks;
+  if (kRouted) {
+    const dsa_const_i32 rp = (dsa_const_i32)p.row_ptr;
+    const int rb = p.route_batches == 1 ? 0 : b;
+    const int64_t csr_row = ((int64_t)rb * p.heads + h) * p.q_blocks + qb;
+    start = rp[csr_row];
+    end = rp[csr_row + 1];
+  }
   if (split) {
     const int n = end - start;
     end = start + (int)((int64_t)n * (part + 1) / p.parts);
@@ -91,7 +98,7 @@ __global__ void __launch_bounds__(128, 2) bsa_fwd_narrow_kernel(BsaParams p) {
   const int nblk = end - start;
   int rot = 0;
   uint64_t* walk_at = nullptr;
-  if (!split && p.walk != nullptr) {
+  if (kRouted && !split && p.walk != nullptr) {
     uint64_t* const tab = p.walk + xcc_id() * kWalkSlots;
     if (nblk > 1) {
       if (wave == 0) {
@@ -173,7 +180,8 @@ __global__ void __launch_bounds__(128, 2) bsa_fwd_narrow_kernel(BsaParams p) {
   const std::bool_constant<false> of_k;
   const std::bool_constant<true> of_v;
   auto gblock = [&](int j) -> int {
-    const int kb = cidx[walked(j < nblk ? j : nblk - 1)];
+    const int at = walked(j < nblk ? j : nblk - 1);
+    const int kb = kRouted ? cidx[at] : at;
     return (unsigned)kb < (unsigned)p.kv_blocks ? kb : -1;
   };
 
@@ -340,13 +348,17 @@ __global__ void __launch_bounds__(128, 2) bsa_fwd_narrow_kernel(BsaParams p) {
     // Stream tile j has ended: its parity's lanes write their rows' entries.
     auto close = [&](int j) __attribute__((always_inline)) {
       if (q4 != (j & 1)) return;
+      // Routed: CSR entry e at e block + row; dense: key tile e of head h at
+      // (h tiles + e) q_tokens + token.
       const int64_t e = walked(j);
-      const bool in = e < p.rs_entries;
+      const bool in = !kRouted || e < p.rs_entries;
+      const int64_t at0 = kRouted ? e * p.block
+                                  : ((int64_t)h * p.kv_blocks + e) * p.q_tokens + qb * p.block;
 #pragma unroll
       for (int n = 0; n < kGroups; ++n) {
         const float mass = carry[n][0];
         if (row_ok[n] && in) {
-          const int64_t at = e * p.block + 16 * (grp0 + n) + c16;
+          const int64_t at = at0 + 16 * (grp0 + n) + c16;
           p.rs_logm[at] = mass > 0.f ? __log2f(mass) + m_run[n] : -INFINITY;
           if (p.rs_mean != nullptr) {
             const float inv = mass > 0.f ? __builtin_amdgcn_rcpf(mass) : 0.f;
@@ -468,7 +480,7 @@ __global__ void __launch_bounds__(128, 2) bsa_fwd_narrow_kernel(BsaParams p) {
   else run(two, kNarrowGroups);
 }
 
-// Routed whole blocks of 65..96 tokens, K and V of one head within 2 GiB.
+// Whole blocks of 65..96 tokens, K and V of one head within 2 GiB.
 inline bool use_narrow(int32_t block, int32_t kv_tokens, int64_t k_token_stride,
                        int64_t v_token_stride) {
   if (block <= kHalfKeys || block > 96 || kv_tokens % block != 0) return false;

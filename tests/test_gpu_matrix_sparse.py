@@ -446,6 +446,41 @@ def test_small_tiles_at_scale(ops, cuda_device, tile_shape, tiles):
             assert metrics["cosine_similarity"] >= 0.9995, (h, qt, metrics)
 
 
+@pytest.mark.parametrize("tile_shape,tiles,dtype", [
+    ((5, 13), 150, torch.bfloat16), ((8, 10), 140, torch.float16), ((9, 9), 140, torch.bfloat16),
+    ((5, 19), 130, torch.float16), ((1, 96), 130, torch.bfloat16)])
+@pytest.mark.parametrize("routed", [True, False])
+def test_narrow_tiles_statistics(ops, cuda_device, tile_shape, tiles, dtype, routed):
+    """Tiles of 65, 80, 81, 95 and 96 tokens in more than 1,024 workgroups
+    (16-row groups): fused statistics, routed and dense, against the separate
+    passes on every cell."""
+    heads = 8
+    tile = tile_shape[0] * tile_shape[1]
+    generator = torch.Generator(device=cuda_device).manual_seed(tiles + tile)
+    q, k, v = (torch.randn((1, tiles * tile, heads, 128), device=cuda_device,
+                           generator=generator).to(dtype) for _ in range(3))
+    csr = None
+    if routed:
+        route = random_route(heads, tiles, seed=tile, keep=0.6)
+        route[..., 0] = True
+        csr = ops.route_to_csr(route.to(cuda_device), block_size=tile)
+    out, lse, got = ops.bsa_fwd_tile_stats(q, k, v, csr, tile_shape)
+    ref, ref_lse = ops.bsa_fwd(q, k, v, csr, return_lse=True,
+                               block_size=tile if routed else 128, deterministic=True)
+    two_pass = ops.tile_stats(q, k, ref_lse, tile_shape, csr=csr)
+    torch.cuda.synchronize()
+    assert (out.float() - ref.float()).abs().max().item() <= 8e-3
+    np.testing.assert_allclose(lse.cpu().numpy(), ref_lse.cpu().numpy(), atol=1e-4)
+    for name in ("mass", "mass_f16"):
+        np.testing.assert_allclose(got[name].float().cpu().numpy(),
+                                   two_pass[name].float().cpu().numpy(), atol=STAT_ATOL,
+                                   rtol=2e-3, err_msg=name)
+    for name in ("centroid_q_y", "centroid_q_x", "centroid_k_y", "centroid_k_x"):
+        np.testing.assert_allclose(got[name].float().cpu().numpy(),
+                                   two_pass[name].float().cpu().numpy(), atol=CENTROID_ATOL,
+                                   err_msg=name)
+
+
 def test_fused_step_at_720p_tile_shape(ops, cuda_device):
     """The bench's 720p matrix-sparse step shape (9 x 8 tiles, 800 tiles
     per head) at 4 heads: fused statistics against the two-pass statistics on
