@@ -176,6 +176,8 @@ _lib = None
 def load():
     """Load libdsa.so once and bind the signatures; raise if it is missing."""
     global _lib
+    if _lib is not None:  # set once, after every signature is bound
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -214,5 +216,4 @@ def pointer_array(values):
 
 
 def int64_array(values):
-    values = [int(value) for value in values]
     return (_c_i64 * len(values))(*values)
