@@ -90,7 +90,7 @@ int prepare(const void* q, const void* k, const void* v, void* o, int32_t dtype,
   p->drop_thresh = 0;
   p->drop_scale = 1.f;
   p->drop_seed_lo = p->drop_seed_hi = p->drop_offset = 0;
-  p->split_max = nullptr;
+  p->split_ranges = nullptr;
   // Set by the launchers that use them.
   p->order = nullptr;
   p->queue = nullptr;
@@ -111,7 +111,7 @@ int launch(int32_t dtype, BsaParams p, void* scratch, size_t scratch_bytes, hipS
   // fp32 inputs run as split fp16 products where the scratch holds them;
   // without, dropout and head dims above 128 run the fp32-compute kernel (no
   // scratch).
-  if (dtype == DSA_F32 && p.drop_thresh == 0 && p.head_dim <= kHeadDim &&
+  if (dtype == DSA_F32 && p.drop_thresh == 0 && p.head_dim <= kHeadDim && split_takes(p) &&
       scratch_bytes >= split_workspace_bytes((int64_t)p.batch * p.heads, p.kv_tokens))
     return bsa_launch_f32_split(p, scratch, scratch_bytes, stream, who);
   if (dtype == DSA_F32 || p.drop_thresh != 0 || p.head_dim > kHeadDim)

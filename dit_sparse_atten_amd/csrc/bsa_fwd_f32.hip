@@ -1,8 +1,8 @@
 // Attention forward in fp32 arithmetic on the matrix cores (gfx950): dense
 // calls with attention dropout, and calls of head dims 136..256, for every
 // input type; and the float32 calls (fp32 in and out) without a workspace for
-// the split products of bsa_fwd_f32s.hip, or their heads with non-finite or
-// extreme elements.
+// the split products of bsa_fwd_f32s.hip, or their heads that split_scales
+// keeps off them.
 //
 // Replaces, for those calls, the SDPA of the reference's DenseBackend
 // (attention_backends/dense.py:34-47, which computes in the `dtype` it is
@@ -122,8 +122,9 @@ __global__ void __launch_bounds__(256, kD == 128 ? 2 : 1) bsa_fwd_f32_kernel(Bsa
   const int b = bh / p.heads;
   // Heads that bsa_fwd_split_kernel has computed.
   if constexpr (std::is_same<T, float>::value && kD == kHeadDim && !kDropout) {
-    if (p.split_max != nullptr &&
-        split_scales(p.split_max, p.batch * p.heads, bh, p.scale_log2).ok)
+    if (p.split_ranges != nullptr && split_scales(p.split_ranges, p.batch * p.heads, bh,
+                                                  p.scale_log2, p.head_dim, p.kv_tokens)
+                                         .ok)
       return;
   }
 

@@ -16,13 +16,20 @@
 // error of O against float64: 7.3e-7, fp32 kernel 1.15e-6).
 //
 // fp16's range: each head of Q, K and V is scaled by the power of two that
-// takes its largest magnitude into [2^14, 2^15) (f32_absmax_kernel finds it),
-// so the split of an element is exact to 2^-24 of it, or to 2^-40 of the
+// takes its largest magnitude into [2^14, 2^15) (f32_range_kernel finds it),
+// so the split of an element is exact to 2^-23 of it, or to 2^-40 of the
 // head's largest; the scales leave the fp32 accumulators exactly.  The
 // probabilities are computed 2^11 times larger, with the row's reference kept
-// within 2^4 of its largest score, for the same reason.  A head with a
-// non-finite or extreme element (split_scales) is left to the fp32 kernel,
-// launched over the same grid, whose workgroups return at once for the others.
+// within 2^4 of its largest score, for the same reason: to 2^-23, or to 2^-36
+// of the row's largest.  A head with a non-finite or extreme element, or whose
+// dims or tokens differ so much that these absolute parts would show
+// (split_scales), is left to the fp32 kernel, launched over the same grid,
+// whose workgroups return at once for the others.
+//
+// Error of O against float64 over that of the fp32 kernel, N(0,1): 0.87 to 0.38
+// at 128 dims from 33 to 3,600 tokens, 0.99 to 0.38 at 64.  Fewer dims and few
+// keys have few roundings in fp32 (8 dims: 1.7 at 16 tokens, 1.03 at 128, 0.94
+// at 256), and run here only from 256 keys for every row (split_takes).
 //
 // Work per 32-key sub-tile and 32 query rows: 48 MFMAs (24 for S^T, 24 for
 // O^T) beside 16 exps and 16 two-way splits per lane; matrix-core bound.  K
@@ -55,45 +62,85 @@ __device__ __forceinline__ void split8(const dsa_f32x4& a, const dsa_f32x4& b, f
   }
 }
 
-// Largest magnitude of kMaxParts token ranges of every head of Q, K and V:
-// workgroup (part, bh, tensor), 32 lanes per token (4 dims each).
-__global__ void __launch_bounds__(256) f32_absmax_kernel(BsaParams p, uint32_t* parts) {
-  const int part = blockIdx.x, bh = blockIdx.y, t = blockIdx.z;
+// Magnitudes of the token ranges of every head of Q, K and V (split_scales):
+// workgroup (range, bh, tensor), 32 lanes per token (4 dims each).
+__global__ void __launch_bounds__(256) f32_range_kernel(BsaParams p, uint32_t* ranges) {
+  const int part = blockIdx.x, bh = blockIdx.y, t = blockIdx.z, pairs = gridDim.y;
   const int h = bh % p.heads, b = bh / p.heads;
-  const int tokens = t == 0 ? p.q_tokens : p.kv_tokens;
-  const int64_t st = t == 0 ? p.q_st : t == 1 ? p.k_st : p.v_st;
-  const float* base = t == 0   ? static_cast<const float*>(p.q) + b * p.q_sb + h * p.q_sh
-                      : t == 1 ? static_cast<const float*>(p.k) + b * p.k_sb + h * p.k_sh
-                               : static_cast<const float*>(p.v) + b * p.v_sb + h * p.v_sh;
-  const int per = (tokens + kMaxParts - 1) / kMaxParts;
-  const int t0 = part * per, t1 = min(t0 + per, tokens);
+  const int tokens = t == kQMax ? p.q_tokens : p.kv_tokens;
+  const int64_t st = t == kQMax ? p.q_st : t == kKMax ? p.k_st : p.v_st;
+  const float* base = t == kQMax   ? static_cast<const float*>(p.q) + b * p.q_sb + h * p.q_sh
+                      : t == kKMax ? static_cast<const float*>(p.k) + b * p.k_sb + h * p.k_sh
+                                   : static_cast<const float*>(p.v) + b * p.v_sb + h * p.v_sh;
+  const int count = range_count(tokens);
+  const int t0 = part < count ? (int)((int64_t)tokens * part / count) : 0;
+  const int t1 = part < count ? (int)((int64_t)tokens * (part + 1) / count) : 0;
   const int c = threadIdx.x & 31;
-  uint32_t best = 0;
+  // Per lane: the largest of each of its dims, and the smallest over the tokens
+  // of its 8-dim group's largest (lanes c and c ^ 1 share a group).
+  uint32_t dim[4] = {0u, 0u, 0u, 0u}, group = 0xffffffffu;
   if (c * 4 < p.head_dim) {
     for (int i = t0 + (threadIdx.x >> 5); i < t1; i += 8) {
       const dsa_u32x4 x = *reinterpret_cast<const dsa_u32x4*>(base + (int64_t)i * st + c * 4);
+      uint32_t top = 0u;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) best = max(best, x[e] & 0x7fffffffu);
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t m = x[e] & 0x7fffffffu;
+        dim[e] = max(dim[e], m);
+        top = max(top, m);
+      }
+      group = min(group, max(top, (uint32_t)__shfl_xor((int)top, 1)));
     }
   }
+  __shared__ uint32_t part_of[4][32][5];
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) best = max(best, (uint32_t)__shfl_xor((int)best, d));
-  __shared__ uint32_t wave_max[4];
-  if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = best;
+  for (int e = 0; e < 4; ++e) dim[e] = max(dim[e], (uint32_t)__shfl_xor((int)dim[e], 32));
+  group = min(group, (uint32_t)__shfl_xor((int)group, 32));
+  if ((threadIdx.x & 32) == 0) {
+    uint32_t* to = part_of[threadIdx.x >> 6][c];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) to[e] = dim[e];
+    to[4] = group;
+  }
   dsa::lds_barrier();
-  if (threadIdx.x == 0)
-    parts[((int64_t)t * gridDim.y + bh) * kMaxParts + part] =
-        max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3]));
+  if (threadIdx.x >= 32) return;
+  uint32_t best = 0u, low = 0xffffffffu;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    uint32_t m = 0u;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) m = max(m, part_of[w][c][e]);
+    best = max(best, m);
+    if (m != 0u) low = min(low, m);
+  }
+  const bool used = max(best, (uint32_t)__shfl_xor((int)best, 1)) != 0u;
+  if (used)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) low = min(low, part_of[w][c][4]);
+  const uint32_t lanes_used = (uint32_t)__ballot(used);
+#pragma unroll
+  for (int d = 1; d < 32; d <<= 1) {
+    best = max(best, (uint32_t)__shfl_xor((int)best, d));
+    low = min(low, (uint32_t)__shfl_xor((int)low, d));
+  }
+  if (c == 0) {
+    const int64_t at = (int64_t)bh * kMaxParts + part, kind = (int64_t)pairs * kMaxParts;
+    ranges[t * kind + at] = best;
+    if (t == kVMax) {
+      ranges[kVLow * kind + at] = low;
+      ranges[kVUsed * kind + at] = lanes_used;
+    }
+  }
 }
 
 // Scaled split rows of K (z = 0) and V (z = 1): workgroup (64 tokens, bh), 16
 // lanes per token (8 dims each; dims past head_dim are zeros).
 constexpr int kSplitTokens = 64;
-__global__ void __launch_bounds__(256) f32_split_kernel(BsaParams p, const uint32_t* parts,
+__global__ void __launch_bounds__(256) f32_split_kernel(BsaParams p, const uint32_t* ranges,
                                                        unsigned char* planes) {
   const int bh = blockIdx.y, pairs = gridDim.y;
   const bool is_v = blockIdx.z != 0;
-  const SplitScales sc = split_scales(parts, pairs, bh, p.scale_log2);
+  const SplitScales sc = split_scales(ranges, pairs, bh, p.scale_log2, p.head_dim, p.kv_tokens);
   if (!sc.ok) return;
   const int h = bh % p.heads, b = bh / p.heads;
   const float scale = is_v ? sc.v : sc.k;
@@ -127,7 +174,7 @@ __global__ void __launch_bounds__(256) f32_split_kernel(BsaParams p, const uint3
 // other's waits; calls too small to give a CU that many keep two.
 template <bool kRouted, bool kStats, int kWaves, bool kSingle>
 __global__ void __launch_bounds__(kWaves * 64, 2) bsa_fwd_split_kernel(
-    BsaParams p, const uint32_t* parts, const unsigned char* planes) {
+    BsaParams p, const uint32_t* ranges, const unsigned char* planes) {
   typedef dsa::Elem<_Float16> E;
   __shared__ __attribute__((aligned(1024))) unsigned char lds_k0[kKStage];
   __shared__ __attribute__((aligned(1024))) unsigned char lds_k1[kSingle ? 16 : kKStage];
@@ -157,7 +204,7 @@ __global__ void __launch_bounds__(kWaves * 64, 2) bsa_fwd_split_kernel(
   const int h = bh % p.heads;
   const int b = bh / p.heads;
   const int pairs = p.batch * p.heads;
-  const SplitScales sc = split_scales(parts, pairs, bh, p.scale_log2);
+  const SplitScales sc = split_scales(ranges, pairs, bh, p.scale_log2, p.head_dim, p.kv_tokens);
   if (!sc.ok) return;  // every wave alike: the fp32 kernel takes this head
 
   int start = 0, end = p.kv_blocks;
@@ -469,11 +516,17 @@ __global__ void __launch_bounds__(kWaves * 64, 2) bsa_fwd_split_kernel(
   }
 }
 
-// Bytes of the magnitude maxima and the split K and V of `pairs` (batch, head)
+// Bytes of the range magnitudes and the split K and V of `pairs` (batch, head)
 // pairs, rounded up to 256.
 size_t split_workspace_bytes(int64_t pairs, int64_t kv_tokens) {
-  return round256((size_t)(3 * pairs * kMaxParts * (int64_t)sizeof(uint32_t) +
+  return round256((size_t)(kRangeKinds * pairs * kMaxParts * (int64_t)sizeof(uint32_t) +
                            2 * pairs * kv_tokens * kSplitRow));
+}
+
+// Whether a float32 call runs here: at head dims below 64 only where every row
+// attends 256 keys (see the errors above).
+bool split_takes(const BsaParams& p) {
+  return p.head_dim >= 64 || (p.row_ptr == nullptr && p.causal == 0 && p.kv_tokens >= 256);
 }
 
 }  // namespace bsa
@@ -485,13 +538,13 @@ int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, size_t workspace_byt
                          hipStream_t stream, const char* who) {
   using namespace bsa;
   const unsigned pairs = (unsigned)(p.batch * p.heads);
-  uint32_t* parts = static_cast<uint32_t*>(workspace);
+  uint32_t* ranges = static_cast<uint32_t*>(workspace);
   unsigned char* planes = static_cast<unsigned char*>(workspace) +
-                          (size_t)3 * pairs * kMaxParts * sizeof(uint32_t);
-  hipLaunchKernelGGL(f32_absmax_kernel, dim3(kMaxParts, pairs, 3), dim3(256), 0, stream, p, parts);
+                          (size_t)kRangeKinds * pairs * kMaxParts * sizeof(uint32_t);
+  hipLaunchKernelGGL(f32_range_kernel, dim3(kMaxParts, pairs, 3), dim3(256), 0, stream, p, ranges);
   hipLaunchKernelGGL(f32_split_kernel,
                      dim3((unsigned)((p.kv_tokens + kSplitTokens - 1) / kSplitTokens), pairs, 2),
-                     dim3(256), 0, stream, p, parts, planes);
+                     dim3(256), 0, stream, p, ranges, planes);
   const int64_t grid = (int64_t)pairs * p.q_blocks;
   // 2-wave workgroups with two stages put two on a CU, with one stage four:
   // the latter where the call has more than two per CU.
@@ -510,7 +563,7 @@ int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, size_t workspace_byt
   p.split_from = (int32_t)(grid - split);
   const dim3 blocks((unsigned)(grid - split + (int64_t)split * p.parts));
   auto run = [&](auto kernel, int waves) {
-    hipLaunchKernelGGL(kernel, blocks, dim3((unsigned)waves * 64), 0, stream, p, parts, planes);
+    hipLaunchKernelGGL(kernel, blocks, dim3((unsigned)waves * 64), 0, stream, p, ranges, planes);
   };
   if (p.row_ptr) {
     if (p.rs_logm) {
@@ -534,6 +587,6 @@ int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, size_t workspace_byt
     }
   }
   if (split > 0) launch_merge<float>(p, split, stream);
-  p.split_max = parts;
+  p.split_ranges = ranges;
   return bsa_launch_f32(p, DSA_F32, stream, who);
 }

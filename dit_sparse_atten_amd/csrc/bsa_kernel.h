@@ -108,9 +108,9 @@ struct BsaParams {
   uint32_t drop_thresh;
   float drop_scale;
   uint32_t drop_seed_lo, drop_seed_hi, drop_offset;
-  // The fp32-compute kernel after bsa_fwd_split_kernel: its magnitude maxima
-  // (null: every head is this kernel's).
-  const uint32_t* split_max;
+  // The fp32-compute kernel after bsa_fwd_split_kernel: the magnitudes that
+  // split_scales decides by (null: every head is this kernel's).
+  const uint32_t* split_ranges;
 };
 
 // One split partial: O [128 rows][128 dims] relative to the row's reference
@@ -1437,4 +1437,5 @@ int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, size_t workspace_byt
                          hipStream_t stream, const char* who);
 namespace bsa {
 size_t split_workspace_bytes(int64_t pairs, int64_t kv_tokens);
+bool split_takes(const BsaParams& p);
 }

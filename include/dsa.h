@@ -123,10 +123,16 @@ size_t dsa_bsa_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
 
 /* Workspace bytes with which an fp32 call of head dim up to 128 (dsa_bsa_fwd;
  * dsa_bsa_fwd_tile_stats and dsa_bsa_fwd_block_mass: beyond their own) runs
- * every fp32 product as three fp16 products on the 16-bit matrix cores, at no
- * larger error (a head with non-finite or extreme elements keeps the fp32
- * products): the split K and V, 1,024 bytes per token, batch item and head, and
- * 768 per batch item and head (rounded up to 256), then 68,157,440 for a split
+ * every fp32 product as three fp16 products on the 16-bit matrix cores.  An
+ * operand is then held to one unit in its last place, or to 2^-40 of its head's
+ * largest magnitude, and the heads where that is too coarse keep the fp32
+ * products: non-finite or extreme elements; Q and K whose magnitudes allow
+ * scores far above those of normalised heads; V with dims, or tokens within a
+ * group of 8 dims, below 2^-12 of the head's largest.  So do head dims below 64
+ * where a row may attend fewer than 256 keys.  On N(0,1) inputs the error
+ * against float64 is 0.4 to 1.0 times that of the fp32 products.
+ * The split K and V take 1,024 bytes per token, batch item and head, and 1,280
+ * per batch item and head (rounded up to 256), then 68,157,440 for a split
  * last round (optional).  0 above head dim 128.  With less workspace the fp32
  * kernel runs. */
 size_t dsa_bsa_f32_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,

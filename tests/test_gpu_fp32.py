@@ -10,6 +10,7 @@ rounding: outputs within 2e-5 of the float64 closed form (values of order
 one), LSE within 2e-5, statistics within rtol 1e-5.
 """
 
+import functools
 import math
 
 import numpy as np
@@ -148,6 +149,108 @@ def test_fp32_split_error_is_no_larger(ops, cuda_device, monkeypatch, tokens, ro
         out = ops.bsa_fwd(q, k, v, csr)[0].double()
         errors.append(((out - exact).norm() / exact.norm()).item())
     assert errors[0] <= errors[1] <= 1e-5, errors
+
+
+def _dense_float64(q, k, v):
+    """O [T, H, D] in float64 (torch, on the device)."""
+    s = (q[0].double().transpose(0, 1) @ k[0].double().permute(1, 2, 0).contiguous())
+    p = torch.softmax(s * q.shape[-1] ** -0.5, dim=-1)
+    return (p @ v[0].double().transpose(0, 1).contiguous()).transpose(0, 1)
+
+
+def _sink(q, k, strength):
+    """Token 7 of head 1 takes a row's attention e^(8 strength / sqrt(128)) times
+    over any other."""
+    q[:, :, 1, 0] = 8
+    k[:, :, 1, 0] = 0
+    k[:, 7, 1, 0] = strength
+
+
+def _spread_inputs(kind, power, q, k, v):
+    """Gives head 1 dims or tokens of very different magnitudes; returns the
+    first output dim to compare."""
+    if kind == "v_dim":
+        v[:, :, 1, 0] *= 2.0 ** power
+        return 1
+    if kind == "qk_dim":
+        k[:, :, 1, 0] *= 2.0 ** power
+        q[:, :, 1, 0] *= 2.0 ** -power
+    elif kind == "k_dim":
+        k[:, :, 1, 0] *= 2.0 ** power
+    elif kind == "q":
+        q[:, :, 1] *= 2.0 ** power
+    elif kind == "v_tokens":  # in every range of tokens, and given no attention
+        q[:, :, 1, 0] = 8
+        k[:, :, 1, 0] = 0
+        k[:, ::8, 1, 0] = -40
+        v[:, ::8, 1] *= 2.0 ** power
+    elif kind == "v_tokens_dims":  # even tokens large in dim 0, odd ones in the others
+        q[:, :, 1, 0] = 8
+        k[:, :, 1, 0] = 0
+        k[:, 1::2, 1, 0] = -40
+        v[:, ::2, 1, 0] *= 2.0 ** power
+        v[:, 1::2, 1, 1:] *= 2.0 ** power
+        return 8
+    elif kind == "sink":
+        _sink(q, k, 26)
+        v[:, 7, 1] *= 2.0 ** power
+    elif kind == "sink_zero":
+        _sink(q, k, 26)
+        v[:, 7, 1] = 0
+    elif kind == "sink_one_dim":
+        _sink(q, k, 30)
+        v[:, 7, 1, 1:] *= 2.0 ** power
+        return 8
+    elif kind == "zero_dims":  # 64 dims used of 128: exact zeros, which cost nothing
+        for x in (q, k, v):
+            x[:, :, 1, 64:] = 0
+    return 0
+
+
+@pytest.mark.parametrize("kind,power,split", [
+    ("v_dim", 6, True), ("v_dim", 18, False), ("v_dim", 24, False), ("v_dim", 38, False),
+    ("qk_dim", 6, True), ("qk_dim", 20, False), ("qk_dim", 24, False),
+    ("k_dim", 6, True), ("k_dim", 16, False), ("q", 5, True), ("q", 11, False),
+    ("v_tokens", 6, True), ("v_tokens", 28, False), ("v_tokens_dims", 24, False),
+    ("sink", -6, True), ("sink", -14, False), ("sink_zero", 0, False),
+    ("sink_one_dim", -30, False), ("zero_dims", 0, True)])
+@pytest.mark.parametrize("tokens", [256, 1100])
+def test_fp32_split_error_on_spread_inputs(ops, cuda_device, monkeypatch, tokens, kind, power,
+                                           split):
+    """Finite heads whose dims or tokens differ widely: the error of O against
+    float64 is at most that of the fp32 products, over the dims that are not the
+    large ones.  ``split``: whether the head runs on the split products (the
+    other head always does)."""
+    q, k, v = (x.to(cuda_device) for x in _qkv(1, tokens, tokens, 2, 128, seed=tokens))
+    first = _spread_inputs(kind, power, q, k, v)
+    exact = _dense_float64(q, k, v)[:, 1, first:]
+    got = ops.bsa_fwd(q, k, v)[0]
+    monkeypatch.setattr(ops, "_f32_workspace_bytes", lambda *args: 0)
+    want = ops.bsa_fwd(q, k, v)[0]
+    assert not torch.equal(got[:, 0], want[:, 0])
+    assert torch.equal(got[:, 1], want[:, 1]) != split
+    errors = [((x[:, 1, first:].double() - exact).norm() / exact.norm()).item()
+              for x in (got, want)]
+    assert errors[0] <= errors[1], errors
+
+
+@pytest.mark.parametrize("tokens,head_dim,causal,routed,split", [
+    (160, 8, False, False, False), (256, 8, False, False, True), (600, 8, True, False, False),
+    (1024, 32, False, True, False), (256, 64, False, True, True), (256, 64, True, False, True)])
+def test_fp32_split_error_of_short_rows(ops, cuda_device, monkeypatch, tokens, head_dim, causal,
+                                        routed, split):
+    """Head dims below 64 keep the fp32 products unless every row attends 256
+    keys: with fewer their error is the smaller one."""
+    q, k, v = (x.to(cuda_device) for x in _qkv(1, tokens, tokens, 2, head_dim, seed=tokens))
+    csr = None
+    if routed:
+        csr = ops.route_to_csr(random_route(2, tokens // 32, seed=3, keep=0.5).to(cuda_device),
+                               block_size=32)
+    call = functools.partial(ops.bsa_fwd, q, k, v, csr, causal=causal,
+                             block_size=32 if routed else 128)
+    got = call()
+    monkeypatch.setattr(ops, "_f32_workspace_bytes", lambda *args: 0)
+    assert torch.equal(got, call()) != split
 
 
 def _tile_inputs(grid, tile, heads, seed):
