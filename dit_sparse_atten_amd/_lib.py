@@ -63,6 +63,7 @@ SIGNATURES = {
     "dsa_bsa_workspace_bytes": (_c_size, (_c_int, _c_int, _c_int, _c_int)),
     "dsa_bsa_workspace_bytes_block": (_c_size, (_c_int, _c_int, _c_int, _c_int, _c_int)),
     "dsa_bsa_f32_workspace_bytes": (_c_size, (_c_int, _c_int, _c_int, _c_int)),
+    "dsa_bsa_f32_workspace_bytes_block": (_c_size, (_c_int, _c_int, _c_int, _c_int, _c_int)),
     "dsa_sampled_mass": (_c_int, (
         _c_ptr, _c_ptr, _c_int,                    # q, k, dtype
         ctypes.POINTER(_c_i64),                    # strides[4]

@@ -333,12 +333,20 @@ extern "C" size_t dsa_bsa_workspace_bytes(int32_t batch, int32_t heads, int32_t 
   return dsa_bsa_workspace_bytes_block(batch, heads, kv_tokens, head_dim, 128);
 }
 
-extern "C" size_t dsa_bsa_f32_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
-                                              int32_t head_dim) {
+extern "C" size_t dsa_bsa_f32_workspace_bytes_block(int32_t batch, int32_t heads,
+                                                    int32_t kv_tokens, int32_t head_dim,
+                                                    int32_t block_size) {
   if (batch <= 0 || heads <= 0 || kv_tokens <= 0 || head_dim <= 0 || head_dim > kHeadDim)
     return 0;
+  if (block_size <= 0 || block_size > 128) return 0;
+  const int32_t kv_blocks = (kv_tokens + block_size - 1) / block_size;
   return split_workspace_bytes((int64_t)batch * heads, kv_tokens) +
-         (size_t)kMaxPartGroups * kPartBytes;
+         (split_max_parts(kv_blocks) >= 2 ? (size_t)kMaxPartGroups * kPartBytes : 0);
+}
+
+extern "C" size_t dsa_bsa_f32_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
+                                              int32_t head_dim) {
+  return dsa_bsa_f32_workspace_bytes_block(batch, heads, kv_tokens, head_dim, 128);
 }
 
 extern "C" int dsa_bsa_fwd(const void* q, const void* k, const void* v, void* o,

@@ -552,13 +552,12 @@ int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, size_t workspace_byt
   const bool two = p.block <= 64, single = grid > slots;
   // Split last round: a 4-wave workgroup alone on a CU runs nearly twice as fast
   // as one of two, so a round is one per CU (2-wave ones: two).  3,600 tokens x
-  // 12 heads (348 workgroups, 92 in five parts) 288 -> 242 us; a part keeps at
-  // least four key blocks.
+  // 12 heads (348 workgroups, 92 in five parts) 288 -> 242 us.
   const size_t lead = split_workspace_bytes(pairs, p.kv_tokens);
   p.part = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + lead);
   p.parts = 1;
   const int split = choose_split(
-      grid, two ? slots : slots / 2, std::min(8, p.kv_blocks / 4),
+      grid, two ? slots : slots / 2, split_max_parts(p.kv_blocks),
       std::min<int64_t>((int64_t)((workspace_bytes - lead) / kPartBytes), kMaxPartGroups), &p.parts);
   p.split_from = (int32_t)(grid - split);
   const dim3 blocks((unsigned)(grid - split + (int64_t)split * p.parts));

@@ -68,12 +68,22 @@ def _kernel_view(name, tensor, dtype=None, attention=False):
     return tensor if ok else tensor.contiguous()
 
 
-def _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim):
+def _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim, block_size):
     """Workspace of the float32 attention's split products (0 for the 16-bit
     types and for head dims above 128)."""
     if q.dtype != torch.float32:
         return 0
-    return lib.dsa_bsa_f32_workspace_bytes(batch, heads, kv_tokens, head_dim)
+    return lib.dsa_bsa_f32_workspace_bytes_block(batch, heads, kv_tokens, head_dim, block_size)
+
+
+def _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, block_size):
+    """Workspace of an attention call with statistics: ``own`` bytes, in which
+    the float32 split products take the place of the 16-bit kernels' scratch."""
+    more = _f32_workspace_bytes(lib, q, 1, heads, tokens, head_dim, block_size)
+    if more:
+        own += max(0, more - lib.dsa_bsa_workspace_bytes_block(1, heads, tokens, head_dim,
+                                                               block_size))
+    return own
 
 
 class RouteCSR:
@@ -224,7 +234,8 @@ def bsa_fwd(q, k, v, csr=None, scale=None, out=None, return_lse=False, block_siz
     # (head dims above 128 run the fp32-compute kernel, which uses none); the
     # caching allocator recycles it.
     if q.dtype == torch.float32 or head_dim > HEAD_DIM:
-        workspace_bytes = _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim)
+        workspace_bytes = _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim,
+                                               block_size)
     else:
         workspace_bytes = lib.dsa_bsa_workspace_bytes_block(
             batch, heads, kv_tokens, head_dim, block_size)
@@ -362,8 +373,9 @@ def bsa_fwd_block_mass(q, k, v, scale=None):
     strides = _lib.int64_array(
         list(q.stride()[:3]) + list(k.stride()[:3]) + list(v.stride()[:3])
         + list(out.stride()[:3]))
-    workspace_bytes = lib.dsa_bsa_fwd_block_mass_workspace_bytes(heads, tokens, head_dim)
-    workspace_bytes += _f32_workspace_bytes(lib, q, 1, heads, tokens, head_dim)
+    workspace_bytes = _statistics_workspace_bytes(
+        lib, q, lib.dsa_bsa_fwd_block_mass_workspace_bytes(heads, tokens, head_dim), heads, tokens,
+        head_dim, 128)
     workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device)
                  if workspace_bytes else None)
     with torch.cuda.device(q.device):
@@ -492,9 +504,10 @@ def bsa_fwd_tile_stats(q, k, v, csr, tile_shape, scale=None, deterministic=False
     strides = _lib.int64_array(
         list(q.stride()[:3]) + list(k.stride()[:3]) + list(v.stride()[:3])
         + list(out.stride()[:3]))
-    workspace_bytes = lib.dsa_bsa_fwd_tile_stats_workspace_bytes(
-        heads, tokens, head_dim, tile_h, tile_w, entries)
-    workspace_bytes += _f32_workspace_bytes(lib, q, 1, heads, tokens, head_dim)
+    workspace_bytes = _statistics_workspace_bytes(
+        lib, q, lib.dsa_bsa_fwd_tile_stats_workspace_bytes(heads, tokens, head_dim, tile_h, tile_w,
+                                                           entries),
+        heads, tokens, head_dim, tile)
     workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device)
                  if workspace_bytes else None)
     with torch.cuda.device(q.device):

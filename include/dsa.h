@@ -121,8 +121,13 @@ int dsa_bsa_fwd(const void* q, const void* k, const void* v, void* o, int32_t dt
 size_t dsa_bsa_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
                                int32_t head_dim);
 
+/* The same for any block_size in 1..128 (key blocks of block_size tokens). */
+size_t dsa_bsa_workspace_bytes_block(int32_t batch, int32_t heads, int32_t kv_tokens,
+                                     int32_t head_dim, int32_t block_size);
+
 /* Workspace bytes with which an fp32 call of head dim up to 128 (dsa_bsa_fwd;
- * dsa_bsa_fwd_tile_stats and dsa_bsa_fwd_block_mass: beyond their own) runs
+ * dsa_bsa_fwd_tile_stats and dsa_bsa_fwd_block_mass: in the place of the
+ * dsa_bsa_workspace_bytes_block bytes within their own) runs
  * every fp32 product as three fp16 products on the 16-bit matrix cores.  An
  * operand is then held to one unit in its last place, or to 2^-40 of its head's
  * largest magnitude, and the heads where that is too coarse keep the fp32
@@ -133,14 +138,13 @@ size_t dsa_bsa_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
  * against float64 is 0.4 to 1.0 times that of the fp32 products.
  * The split K and V take 1,024 bytes per token, batch item and head, and 1,280
  * per batch item and head (rounded up to 256), then 68,157,440 for a split
- * last round (optional).  0 above head dim 128.  With less workspace the fp32
- * kernel runs. */
+ * last round (optional) when the key range holds at least 8 blocks (two parts
+ * of at least 4 key blocks).  0 above head dim 128.  With less workspace the
+ * fp32 kernel runs.  _block: for any block_size in 1..128. */
 size_t dsa_bsa_f32_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
                                    int32_t head_dim);
-
-/* The same for any block_size in 1..128 (key blocks of block_size tokens). */
-size_t dsa_bsa_workspace_bytes_block(int32_t batch, int32_t heads, int32_t kv_tokens,
-                                     int32_t head_dim, int32_t block_size);
+size_t dsa_bsa_f32_workspace_bytes_block(int32_t batch, int32_t heads, int32_t kv_tokens,
+                                         int32_t head_dim, int32_t block_size);
 
 /*
  * dsa_bsa_fwd without a workspace argument, for callers that cannot allocate

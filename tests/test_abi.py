@@ -64,6 +64,22 @@ def test_version_and_workspace_size(lib):
     assert lib.dsa_bsa_workspace_bytes(0, 12, 10, 128) == 0
 
 
+def test_f32_workspace_size(lib):
+    # 64 magnitudes of five kinds per (batch, head), the split K and V (128 hi
+    # and 128 lo fp16 values per token each), then the split partials when the
+    # key range can be split (at least 8 key blocks, 2 parts of 4).
+    def planes(pairs, tokens):
+        return pairs * (5 * 64 * 4 + 2 * tokens * 512)
+
+    split = 1024 * (128 * 128 + 256) * 4
+    assert lib.dsa_bsa_f32_workspace_bytes(1, 12, 512, 128) == planes(12, 512)
+    assert lib.dsa_bsa_f32_workspace_bytes(2, 12, 897, 64) == planes(24, 897) + split
+    assert lib.dsa_bsa_f32_workspace_bytes_block(1, 12, 512, 128, 64) == planes(12, 512) + split
+    assert lib.dsa_bsa_f32_workspace_bytes_block(1, 3, 504, 128, 72) == planes(3, 504)
+    assert lib.dsa_bsa_f32_workspace_bytes(1, 12, 512, 136) == 0
+    assert lib.dsa_bsa_f32_workspace_bytes_block(1, 12, 512, 128, 129) == 0
+
+
 def test_invalid_arguments_are_reported_before_any_launch(lib):
     strides = _lib.int64_array([8] * 12)
     status = lib.dsa_bsa_fwd(None, None, None, None, 0, strides, 1, 128, 128, 1, 128, 128,

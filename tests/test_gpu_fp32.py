@@ -312,6 +312,26 @@ def test_fp32_tile_step_matches_oracle(ops, cuda_device, routed, grid, tile):
         assert (got["mass"].cpu().numpy()[~route] == 0).all()
 
 
+def test_fp32_statistics_take_one_scratch(ops, cuda_device):
+    """The workspace of a float32 call with statistics holds the row statistics
+    and the split products' scratch, not the 16-bit kernels' beside them: 2,048
+    tokens x 2 heads in 8 x 8 tiles, peak memory of the call."""
+    tokens, heads, tiles = 2048, 2, 32
+    q, k, v = (x.to(cuda_device) for x in _qkv(1, tokens, tokens, heads, 128, seed=1))
+    for call, rows in ((lambda: ops.bsa_fwd_tile_stats(q, k, v, None, (8, 8)),
+                        8 * tiles * tiles * 64),
+                       (lambda: ops.bsa_fwd_block_mass(q, k, v), 4 * 16 * 16 * 128)):
+        call()
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        outputs = call()  # noqa: F841 (held while the peak is read)
+        peak = torch.cuda.max_memory_allocated() - before
+        split = heads * (5 * 64 * 4 + 2 * tokens * 512) + 1024 * (128 * 128 + 256) * 4
+        out = 4 * tokens * heads * 129 + heads * tiles * tiles * 14
+        assert peak <= split + heads * rows + out + (4 << 20), peak
+
+
 def test_fp32_block_mass_matches_float64(ops, cuda_device):
     """The exact 128-token block mass of a float32 dense call (the flex
     backend's exact bootstrap) against the float64 closed form."""
