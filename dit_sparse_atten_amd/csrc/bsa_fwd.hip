@@ -108,11 +108,14 @@ int prepare(const void* q, const void* k, const void* v, void* o, int32_t dtype,
 // (launch order, then split partials; see launch_typed).
 int launch(int32_t dtype, BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t stream,
            const char* who) {
-  // fp32 inputs run as split fp16 products where the scratch holds them;
-  // without, dropout and head dims above 128 run the fp32-compute kernel (no
-  // scratch).
+  // fp32 inputs run as split fp16 products where the caller has given the scratch
+  // of dsa_bsa_f32_workspace_bytes_block; without, dropout and head dims above 128
+  // run the fp32-compute kernel (no scratch).  The partials that a split may
+  // use are required with it: so the scratch of the 16-bit kernels, 68 MB from 16
+  // key blocks on, never passes for it.
   if (dtype == DSA_F32 && p.drop_thresh == 0 && p.head_dim <= kHeadDim && split_takes(p) &&
-      scratch_bytes >= split_workspace_bytes((int64_t)p.batch * p.heads, p.kv_tokens))
+      scratch_bytes >= dsa_bsa_f32_workspace_bytes_block(p.batch, p.heads, p.kv_tokens, p.head_dim,
+                                                         p.block))
     return bsa_launch_f32_split(p, scratch, scratch_bytes, stream, who);
   if (dtype == DSA_F32 || p.drop_thresh != 0 || p.head_dim > kHeadDim)
     return bsa_launch_f32(p, dtype, stream, who);
@@ -389,7 +392,8 @@ extern "C" int dsa_bsa_fwd_noalloc(const void* q, const void* k, const void* v, 
   // Calls of more work items than the order region holds run in launch
   // order, as dsa_bsa_fwd does; the split never takes more partials than the
   // array holds.  So no call size needs more scratch than this.
-  // fp32 calls keep to the kernel that takes none, so they may overlap.
+  // fp32 calls keep to the kernel that takes none, so they may overlap; so does
+  // dsa_bsa_fwd with the scratch of the 16-bit kernels.
   return launch(dtype, p, area, dtype == DSA_F32 ? 0 : kScratchBytes, stream,
                 "dsa_bsa_fwd_noalloc");
 }

@@ -43,7 +43,9 @@ const char* dsa_last_error(void);
  * Block-sparse attention forward, bf16, fp16 or fp32 in and out (dtype), fp32
  * online softmax; the matrix products run in the input type with fp32
  * accumulation (fp32 inputs: fp32 products on v_mfma_f32_32x32x2_f32, the
- * probabilities unrounded).
+ * probabilities unrounded; with a workspace of at least
+ * dsa_bsa_f32_workspace_bytes_block() bytes split fp16 products, see there, and
+ * with less, that of dsa_bsa_workspace_bytes_block() included, never).
  * Replaces FlexAttention over a BlockMask (attention_backends/flex.py:379-399
  * `_flex_output`, flex.py:360-376) and, with row_ptr == col_idx == NULL, dense
  * SDPA (attention_backends/dense.py:14-48).
@@ -139,8 +141,9 @@ size_t dsa_bsa_workspace_bytes_block(int32_t batch, int32_t heads, int32_t kv_to
  * The split K and V take 1,024 bytes per token, batch item and head, and 1,280
  * per batch item and head (rounded up to 256), then 68,157,440 for a split
  * last round (optional) when the key range holds at least 8 blocks (two parts
- * of at least 4 key blocks).  0 above head dim 128.  With less workspace the
- * fp32 kernel runs.  _block: for any block_size in 1..128. */
+ * of at least 4 key blocks).  0 above head dim 128.  With less workspace
+ * (always more than dsa_bsa_workspace_bytes_block() bytes) the fp32 kernel
+ * runs, so the workspace a caller gives is the choice between the two.  _block: for any block_size in 1..128. */
 size_t dsa_bsa_f32_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,
                                    int32_t head_dim);
 size_t dsa_bsa_f32_workspace_bytes_block(int32_t batch, int32_t heads, int32_t kv_tokens,
@@ -151,7 +154,8 @@ size_t dsa_bsa_f32_workspace_bytes_block(int32_t batch, int32_t heads, int32_t k
  * device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  No counterpart in the reference.  Same arguments,
  * semantics and results as dsa_bsa_fwd given a workspace of
- * dsa_bsa_workspace_bytes_block() bytes; it calls no hipMalloc / hipFree.  The
+ * dsa_bsa_workspace_bytes_block() bytes (fp32 calls: fp32 products, which take
+ * no scratch); it calls no hipMalloc / hipFree.  The
  * work queue, the launch order, the aligned-walk positions, the key-norm
  * maxima and the split partials live in a library-owned device array of
  * 70,258,944 bytes (256 bytes of queue, 1 MiB of order, 4 KiB of positions,

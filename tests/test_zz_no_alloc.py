@@ -72,6 +72,37 @@ def test_noalloc_matches_workspace_entry_point(cuda_device):
                 np.testing.assert_allclose(lse.cpu().numpy(), expected_lse, atol=1e-3, rtol=1e-4)
 
 
+@pytest.mark.parametrize("tokens,heads", [(2048, 2), (3600, 12)])
+def test_noalloc_matches_workspace_entry_point_in_fp32(cuda_device, tokens, heads):
+    """Float32 calls: with the workspace of dsa_bsa_workspace_bytes_block, which
+    holds the split K and V of a call of this size too, the same products as
+    without one, bit for bit; with that of dsa_bsa_f32_workspace_bytes the
+    split products."""
+    from dit_sparse_atten_amd import _lib
+    lib = _lib.load()
+    stream = torch.cuda.current_stream(cuda_device).cuda_stream
+    generator = torch.Generator().manual_seed(tokens)
+    q, k, v = (torch.randn(1, tokens, heads, 128, generator=generator).to(cuda_device)
+               for _ in range(3))
+    outs = []
+    for bytes_ in (None, lib.dsa_bsa_workspace_bytes(1, heads, tokens, 128),
+                   lib.dsa_bsa_f32_workspace_bytes(1, heads, tokens, 128)):
+        out, lse = torch.empty_like(q), torch.empty((1, heads, tokens), device=cuda_device)
+        args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _lib.DSA_DTYPE_F32,
+                _strides(q, k, v, out), 1, tokens, tokens, heads, 128, 128, None, None, 1,
+                128 ** -0.5, 0, 1, lse.data_ptr())
+        if bytes_ is None:
+            _lib.check(lib.dsa_bsa_fwd_noalloc(*args, stream), "dsa_bsa_fwd_noalloc")
+        else:
+            workspace = torch.empty(bytes_, dtype=torch.uint8, device=cuda_device)
+            _lib.check(lib.dsa_bsa_fwd(*args, workspace.data_ptr(), bytes_, stream), "dsa_bsa_fwd")
+        torch.cuda.synchronize()
+        outs.append((out, lse))
+    for got, want in zip(outs[1], outs[0]):
+        assert torch.equal(got, want)
+    assert not torch.equal(outs[2][0], outs[0][0])
+
+
 def test_noalloc_validates_before_launch(cuda_device):
     from dit_sparse_atten_amd import _lib
     lib = _lib.load()
