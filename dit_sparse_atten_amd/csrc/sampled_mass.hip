@@ -306,17 +306,20 @@ __global__ void __launch_bounds__(256, kHalves == 1 ? 3 : 2) sampled_mass_kernel
         };
         float sum = terms();
         if (__any(!(sum <= kMoveSum))) {
-          // Some row's terms have outgrown its reference (or are not finite):
-          // move the reference to the row's largest score.
+          // Rows whose terms have outgrown their reference move it to their
+          // largest score; both lanes of a row alike.  (A NaN row never does, and
+          // must not have the wave rewrite its sums on every sub-tile.)
           const float mx = row_max();
-          const bool up = mx > m2;
-          const float alpha = up ? __builtin_amdgcn_exp2f(m2 - mx) : 1.f;
-          if (up) m2 = mx;
-          l2 *= alpha;
-          settle_part();
-          for (int kb = g; kb < kb0; kb += 2) part[kb * 32 + qi] *= alpha;
-          settle_part();
-          sum = terms();
+          const bool up = mx > m2 && dsa::pair32_max(sum) > kMoveSum;
+          if (__any(up)) {
+            const float alpha = up ? __builtin_amdgcn_exp2f(m2 - mx) : 1.f;
+            if (up) m2 = mx;
+            l2 *= alpha;
+            settle_part();
+            for (int kb = g; kb < kb0; kb += 2) part[kb * 32 + qi] *= alpha;
+            settle_part();
+            sum = terms();
+          }
         }
         l2 += sum;
         if constexpr (SP >= 8 && kOwn > 1) {

@@ -141,6 +141,37 @@ def test_sampled_mass_one_sweep_non_finite_rows(ops, cuda_device):
     torch.testing.assert_close(got, want, rtol=2.5e-4, atol=1e-9, equal_nan=True)
 
 
+def test_sampled_mass_non_finite_row_costs_no_rescans(ops, cuda_device):
+    """A NaN query row stays NaN for the whole scan; its wave must not rewrite
+    its earlier sums for it on every sub-tile, which is quadratic in the blocks
+    (28,800 tokens x 8 heads, one such row per head; device time, best of 5)."""
+    tokens, heads = 28800, 8
+    generator = torch.Generator(device=cuda_device).manual_seed(2)
+    q, k = (torch.randn(1, tokens, heads, 128, device=cuda_device, generator=generator)
+            .bfloat16() for _ in range(2))
+    bad = q.clone()
+    bad[0, 128 + 4] = float("nan")
+
+    def best(query):
+        times = []
+        for _ in range(5):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(10):
+                ops.sampled_block_mass(query, k, 128, 16)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    want, got = ops.sampled_block_mass(q, k, 128, 16), ops.sampled_block_mass(bad, k, 128, 16)
+    assert got[:, 1].isnan().all()
+    others = torch.arange(got.shape[1], device=cuda_device) != 1
+    assert torch.equal(got[:, others], want[:, others])
+    plain, odd = best(q), best(bad)
+    assert odd < 1.5 * plain, (plain, odd)
+
+
 def test_sampled_mass_one_sweep_in_several_launches(ops, cuda_device):
     """1,040 workgroups over a workspace of 1,024 slots: two launches."""
     from dit_sparse_atten_amd import _lib
