@@ -38,7 +38,7 @@ struct MassParams {
   float scale;      // score scale (d^-1/2 unless given)
   float logw_full;  // log(block_size / S)
   float logw_last;  // log(size of the last block / S)
-  // One-sweep kernel: row-block sums of the launch's workgroups (kRowSlot
+  // One-sweep kernel: row-block sums of the launch's workgroups (kGroupRows
   // floats per key block and workgroup), and the launch's first workgroup.
   float* part;
   int32_t first, row_tiles;  // row_tiles: 128-row workgroups per head
@@ -571,12 +571,14 @@ int sample_stride(int32_t samples) {
   return sp;
 }
 
-// One-sweep workspace: a slot of row sums per workgroup, for the smaller of
-// every workgroup and kMinSlots or what kSlotBytes holds; larger calls run in
-// several launches over the same slots.  kMinSlots is what the chip holds at
-// once (four workgroups of 32 KB LDS per CU), so a launch of fewer would idle
-// CUs.
-constexpr int64_t kMinSlots = 1024;
+// One-sweep workspace: a slot of row sums per workgroup, for every workgroup or
+// as many chip-fulls as kSlotBytes holds, and at least one; a call of more runs in
+// launches of whole chip-fulls over the same slots.  A CU holds three of the
+// kernel's workgroups (four waves each, three per SIMD), two above head dim 128.
+// (57,600 tokens x 40 heads, 16 samples, 2,280 workgroups: 598 MB in one launch,
+// 1,042 us; in launches of two chip-fulls 1,056 us, of one 1,060.  Workgroups that
+// stay and take one group after the other are no faster than launches of one.)
+constexpr int64_t kChipGroups = 3 * 256, kChipGroupsWide = 2 * 256;
 constexpr int64_t kSlotBytes = (int64_t)1 << 30;
 
 int64_t slot_bytes(int64_t blocks) {
@@ -594,8 +596,8 @@ extern "C" size_t dsa_sampled_mass_workspace_bytes(int32_t tokens, int32_t heads
   if (sp > 32) return 0;
   const int64_t blocks = ((int64_t)tokens + block_size - 1) / block_size;
   const int64_t groups = (blocks * sp + kGroupRows - 1) / kGroupRows * heads;
-  const int64_t slots = std::max(kMinSlots, kSlotBytes / slot_bytes(blocks));
-  return (size_t)(std::min(groups, slots) * slot_bytes(blocks));
+  const int64_t chips = std::max<int64_t>(1, kSlotBytes / (kChipGroups * slot_bytes(blocks)));
+  return (size_t)(std::min(groups, chips * kChipGroups) * slot_bytes(blocks));
 }
 
 extern "C" int dsa_sampled_mass(const void* q, const void* k, int32_t dtype,
@@ -667,12 +669,13 @@ extern "C" int dsa_sampled_mass_ws(const void* q, const void* k, int32_t dtype,
   // Padded instances for sample counts that are not a power of two, and for
   // 64 and 128 samples (key and query blocks wider than a sub-tile or wave).
   const bool pad = sp != samples || sp > 32;
-  // One sweep where the workspace holds a chip's worth of row sums.
+  // One sweep where the workspace holds a chip-full of row sums, or all.
   const int64_t slots = std::min<int64_t>(
       groups, workspace ? (int64_t)workspace_bytes / slot_bytes(p.blocks) : 0);
-  const bool once = sp <= 32 && slots >= std::min(groups, kMinSlots);
+  const bool once = sp <= 32 && slots >= std::min(groups, kChipGroups);
   p.part = once ? static_cast<float*>(workspace) : nullptr;
-  const int64_t step = once ? slots : groups;
+  const int64_t chip = head_dim > kHeadDim ? kChipGroupsWide : kChipGroups;
+  const int64_t step = !once || slots == groups ? groups : slots / chip * chip;
   for (int64_t first = 0; first < groups; first += step) {
     p.first = (int32_t)first;
     const int n = (int)std::min(step, groups - first);

@@ -214,8 +214,13 @@ int dsa_sampled_mass(const void* q, const void* k, int32_t dtype, const int64_t*
 
 /*
  * dsa_sampled_mass with a workspace, 16-byte aligned: with at least
- * dsa_sampled_mass_workspace_bytes(...) bytes (0 above 32 samples) every score
- * is computed once instead of twice.  NULL and 0 are allowed.
+ * dsa_sampled_mass_workspace_bytes(...) bytes every score is computed once
+ * instead of twice.  That is, for up to 32 samples (0 above), 512 bytes per key
+ * block (their number rounded up to 64) and workgroup of 128 sampled rows of a
+ * head, of every workgroup, up to 1 GiB (but of 768 always): 598 MB at 57,600 tokens x 40 heads, 16
+ * samples.  Less runs too: with 768 such slots (201 MB there) 2 to 5% slower, in
+ * several launches, and with less (NULL and 0 included) in two scans, about 1.5
+ * times as long.
  */
 int dsa_sampled_mass_ws(const void* q, const void* k, int32_t dtype, const int64_t* strides,
                         int32_t tokens, int32_t heads, int32_t head_dim, int32_t block_size,

@@ -86,6 +86,20 @@ def test_f32_workspace_size(lib):
     assert lib.dsa_bsa_f32_workspace_bytes_block(1, 12, 512, 128, 129) == 0
 
 
+def test_sampled_mass_workspace_size(lib):
+    # A slot per workgroup of 128 sampled rows, 512 bytes per key block (rounded
+    # up to 64); above 1 GiB whole chip-fulls of 768 slots, and one at least.
+    def slot(blocks):
+        return (blocks + 63) // 64 * 64 * 512
+
+    size = lib.dsa_sampled_mass_workspace_bytes
+    assert size(57600, 40, 128, 16) == 40 * 57 * slot(450)
+    assert size(57600, 40, 128, 32) == 5 * 768 * slot(450)  # 4,520 workgroups
+    assert size(1 << 20, 40, 128, 16) == 768 * slot(8192)
+    assert size(1000, 2, 128, 12) == 2 * slot(8)
+    assert size(57600, 40, 128, 33) == 0
+
+
 def test_invalid_arguments_are_reported_before_any_launch(lib):
     strides = _lib.int64_array([8] * 12)
     status = lib.dsa_bsa_fwd(None, None, None, None, 0, strides, 1, 128, 128, 1, 128, 128,

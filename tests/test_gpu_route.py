@@ -196,6 +196,30 @@ def test_sampled_mass_one_sweep_in_several_launches(ops, cuda_device):
     assert torch.equal(mass, want)
 
 
+@pytest.mark.parametrize("dim,slots,once", [(128, 768, True), (128, 767, False),
+                                            (256, 800, True)])
+def test_sampled_mass_one_sweep_in_chip_fulls(ops, cuda_device, dim, slots, once):
+    """1,040 workgroups over a workspace of fewer slots: one sweep, in launches
+    of whole chip-fulls (768, or 512 above head dim 128), from 768 slots on."""
+    from dit_sparse_atten_amd import _lib
+    tokens, heads, samples = 13312, 40, 32
+    generator = torch.Generator(device=cuda_device).manual_seed(3)
+    q, k = (torch.randn((1, tokens, heads, dim), device=cuda_device, generator=generator)
+            .to(torch.bfloat16) for _ in range(2))
+    want = ops.sampled_block_mass(q, k, 128, samples) if once else _two_sweep_mass(q, k, 128,
+                                                                                  samples)
+    workspace = torch.empty(slots * 128 * 512, dtype=torch.uint8, device=cuda_device)
+    mass = torch.empty_like(want)
+    strides = _lib.int64_array([q.stride(1), q.stride(2), k.stride(1), k.stride(2)])
+    status = _lib.load().dsa_sampled_mass_ws(
+        q.data_ptr(), k.data_ptr(), 0, strides, tokens, heads, dim, 128, samples, dim ** -0.5,
+        mass.data_ptr(), workspace.data_ptr(), workspace.numel(),
+        torch.cuda.current_stream().cuda_stream)
+    _lib.check(status, "dsa_sampled_mass_ws")
+    torch.cuda.synchronize()
+    assert torch.equal(mass, want)
+
+
 def test_full_sampling_at_block_128_matches_exact_block_mass(ops, cuda_device):
     """samples == block == 128 (the reference's identity, test_flex_backend.py:
     43-53, at the production block size): mass = exact mass / block, up to
