@@ -547,12 +547,17 @@ extern "C" int dsa_bsa_fwd_block_mass(const void* q, const void* k, const void* 
   if (status != DSA_OK) return status;
   if (workspace_bytes > 0 && (!workspace || !aligned16(workspace)))
     return dsa::set_error(DSA_EINVAL, "%s: workspace must be 16-byte aligned", who);
-  const size_t need = dsa_bsa_fwd_block_mass_workspace_bytes(heads, tokens, head_dim);
+  // A partial last block also runs on the attention's scratch alone, in two
+  // passes: its row sums take heads * blocks^2 * 512 bytes (4.2 GB at 57,601
+  // tokens x 40 heads).
+  const size_t full = dsa_bsa_fwd_block_mass_workspace_bytes(heads, tokens, head_dim);
+  const size_t need =
+      tokens % 128 != 0 ? dsa_bsa_workspace_bytes(1, heads, tokens, head_dim) : full;
   if (workspace_bytes < need)
     return dsa::set_error(DSA_EINVAL, "%s: workspace of %zu bytes, %zu needed", who,
                           workspace_bytes, need);
   unsigned char* base = static_cast<unsigned char*>(workspace);
-  if (mass_pass(tokens, head_dim)) {
+  if (mass_pass(tokens, head_dim) || workspace_bytes < full) {
     status = launch(dtype, p, base, workspace_bytes, stream, who);
     if (status != DSA_OK) return status;
     const int64_t mass_strides[4] = {strides[1], strides[2], strides[4], strides[5]};

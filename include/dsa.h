@@ -327,13 +327,16 @@ size_t dsa_bsa_fwd_tile_stats_workspace_bytes(int32_t heads, int32_t tokens, int
  *   workspace: dsa_bsa_fwd_block_mass_workspace_bytes(...) bytes, 16-byte
  *            aligned: heads * blocks^2 * 128 * 4 bytes of per-row log-masses
  *            when fused (rounded up to 256), then dsa_bsa_fwd's workspace.
+ *            With tokens not a multiple of 128 the latter alone
+ *            (dsa_bsa_workspace_bytes(1, heads, tokens, head_dim)) is enough:
+ *            the call then runs the attention and then dsa_block_mass.
  */
 int dsa_bsa_fwd_block_mass(const void* q, const void* k, const void* v, void* o, int32_t dtype,
                            const int64_t* strides, int32_t tokens, int32_t heads,
                            int32_t head_dim, float scale, float* lse, float* mass,
                            void* workspace, size_t workspace_bytes, hipStream_t stream);
 
-/* Workspace bytes dsa_bsa_fwd_block_mass needs (0 for invalid sizes).  No
+/* Workspace bytes of a fused dsa_bsa_fwd_block_mass (0 for invalid sizes).  No
  * counterpart in the reference. */
 size_t dsa_bsa_fwd_block_mass_workspace_bytes(int32_t heads, int32_t tokens, int32_t head_dim);
 
