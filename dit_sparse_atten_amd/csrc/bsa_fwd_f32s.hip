@@ -524,8 +524,16 @@ size_t split_workspace_bytes(int64_t pairs, int64_t kv_tokens) {
 }
 
 // Whether a float32 call runs here: at head dims below 64 only where every row
-// attends 256 keys (see the errors above).
+// attends 256 keys (see the errors above), and only with enough keys for four
+// launches, each waiting for the one before, to beat one launch of the fp32
+// kernel, whose workgroups take 0.15 us per key.  us here / there, same box:
+// 3,600 queries x 12 heads on 32 keys 32 / 23, 2,400 x 40 on 64 keys 55 / 52; 96
+// keys: 96 tokens x 12 heads 24 / 20 (1,024 queries on 77 keys 28 / 23), but
+// 3,600 queries x 12 heads 37 / 43 and 14,400 x 40 on 77 keys 275 / 319, as the
+// fp32 kernel runs out of CUs; 97 tokens x 12 heads 25 / 25, 256 tokens 32 / 45.
 bool split_takes(const BsaParams& p) {
+  if (p.kv_tokens <= kSplitFewKeys) return false;
+  if (p.kv_tokens <= 96 && (int64_t)p.batch * p.heads * p.q_blocks <= 256) return false;
   return p.head_dim >= 64 || (p.row_ptr == nullptr && p.causal == 0 && p.kv_tokens >= 256);
 }
 

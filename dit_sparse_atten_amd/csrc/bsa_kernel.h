@@ -1437,6 +1437,7 @@ int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, size_t workspace_byt
                          hipStream_t stream, const char* who);
 namespace bsa {
 size_t split_workspace_bytes(int64_t pairs, int64_t kv_tokens);
+constexpr int32_t kSplitFewKeys = 64;  // never taken up to here
 bool split_takes(const BsaParams& p);
 // Parts a query block of its last round may take: at least four key blocks each.
 inline int split_max_parts(int32_t kv_blocks) { return std::min(8, kv_blocks / 4); }

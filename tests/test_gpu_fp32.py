@@ -88,7 +88,8 @@ def test_fp32_routed_matches_float64(ops, cuda_device, tokens, block):
 
 
 @pytest.mark.parametrize("tokens,heads,block,routed", [
-    (33, 8, 128, False), (130, 8, 64, True), (4096, 16, 64, True), (1100, 8, 100, True)])
+    (33, 8, 128, False), (97, 8, 128, False), (130, 8, 64, True), (4096, 16, 64, True),
+    (1100, 8, 100, True)])
 def test_fp32_split_heads_against_fp32_products(ops, cuda_device, monkeypatch, tokens, heads,
                                                 block, routed):
     """Heads of very different magnitudes in one call, with the workspace (split
@@ -96,7 +97,8 @@ def test_fp32_split_heads_against_fp32_products(ops, cuda_device, monkeypatch, t
     heads with non-finite or extreme elements on the fp32 kernel, bit for bit.
     2-wave workgroups with one stage (1,024 of them) and with two, 4-wave ones,
     sub-tiles of 1, 2, 4 and 32 keys, and (1,100 tokens: 88 workgroups, 11 key
-    blocks) every query block in two key ranges."""
+    blocks) every query block in two key ranges.  33 tokens: every head on the
+    fp32 kernel (few keys)."""
     q, k, v = (x.to(cuda_device) for x in _qkv(1, tokens, tokens, heads, 128, seed=tokens))
     q[:, :, 1] *= 2.0 ** 20
     k[:, :, 1] *= 2.0 ** -20
@@ -122,11 +124,26 @@ def test_fp32_split_heads_against_fp32_products(ops, cuda_device, monkeypatch, t
         torch.testing.assert_close(got[:, :, head] / scale, want[:, :, head] / scale,
                                    atol=2 * OUT_ATOL, rtol=0)
         torch.testing.assert_close(got_lse[:, head], want_lse[:, head], atol=2 * LSE_ATOL, rtol=0)
-    assert not torch.equal(got[:, :, 0], want[:, :, 0])  # two different kernels ran
+    # Two different kernels ran, or with few keys the same one.
+    assert torch.equal(got[:, :, 0], want[:, :, 0]) == (tokens == 33)
     for head in range(3, 8):
         assert torch.equal(got[:, :, head].view(torch.int32), want[:, :, head].view(torch.int32))
         assert torch.equal(got_lse[:, head].view(torch.int32),
                            want_lse[:, head].view(torch.int32))
+
+
+@pytest.mark.parametrize("q_tokens,kv_tokens,split", [
+    (64, 64, False), (16500, 64, False), (96, 96, False), (16384, 96, False), (16500, 65, True),
+    (16500, 96, True), (97, 97, True)])
+def test_fp32_few_keys_keep_one_launch(ops, cuda_device, monkeypatch, q_tokens, kv_tokens, split):
+    """Up to 64 keys, and up to 96 with at most 256 query blocks, a float32 call
+    runs the fp32 kernel alone (2 heads: 16,384 queries are 256 blocks)."""
+    q, k, v = (x.to(cuda_device) for x in _qkv(1, q_tokens, kv_tokens, 2, 128, seed=kv_tokens))
+    got = ops.bsa_fwd(q, k, v)
+    monkeypatch.setattr(ops, "_f32_workspace_bytes", lambda *args: 0)
+    want = ops.bsa_fwd(q, k, v)
+    assert torch.equal(got, want) != split
+    torch.testing.assert_close(got, want, atol=2 * OUT_ATOL, rtol=0)
 
 
 @pytest.mark.parametrize("tokens,routed", [(1024, False), (6000, False), (6016, True)])
