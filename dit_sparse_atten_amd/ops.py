@@ -495,9 +495,10 @@ def bsa_fwd_tile_stats(q, k, v, csr, tile_shape, scale=None, deterministic=False
             raise ValueError("route shape does not match the tile layout")
         if csr.row_ptr.device != q.device or csr.col_idx.device != q.device:
             raise ValueError("route must live on the attention device")
-        # Room for every cell where that is little; else for the listed ones, whose
-        # number the device holds (a read that waits for it).
-        entries = heads * tiles * tiles
+        # Room for every entry the list can hold where that is little (a caller's
+        # own list may name a tile twice); else for the listed ones, whose number
+        # the device holds (a read that waits for it).
+        entries = csr.col_idx.numel()
         if entries * tile > MAX_UNCOUNTED_ROWS:
             entries = csr.nnz_value() if csr.nnz is not None else int(csr.row_ptr[-1].item())
     else:

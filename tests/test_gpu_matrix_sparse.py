@@ -170,6 +170,31 @@ def test_routed_tile_stats_skip_out_of_range_tiles(ops, cuda_device):
     _compare_stats(got, expected)
 
 
+@pytest.mark.parametrize("grid,tile", [((2, 18, 32), 64), ((4, 16, 16), 64), ((2, 22, 22), 121)])
+def test_fused_step_of_a_list_longer_than_the_cells(ops, cuda_device, grid, tile):
+    """A caller's CSR that lists every tile and, in each row, three out-of-range
+    ones (which are skipped): more entries than cells, all of whose statistics
+    are kept."""
+    case, q, k, v = _tile_major_inputs(grid, 2, seed=3, tile=tile)
+    tiles = q.shape[1] // case.tile
+    qd, kd, vd = (x.to(cuda_device) for x in (q, k, v))
+    row = torch.cat((torch.tensor([-1, tiles]), torch.arange(tiles), torch.tensor([1 << 20])))
+    rows = 2 * tiles
+    csr = ops.RouteCSR(
+        (torch.arange(rows + 1) * (tiles + 3)).int().to(cuda_device),
+        row.int().repeat(rows).to(cuda_device),
+        torch.full((rows,), tiles + 3, dtype=torch.int32).to(cuda_device), 1, 2, tiles, tiles,
+        case.tile)
+    full = ops.route_to_csr(torch.ones(2, tiles, tiles, dtype=torch.bool, device=cuda_device),
+                            block_size=case.tile)
+    _, lse, got = ops.bsa_fwd_tile_stats(qd, kd, vd, csr, case.tile_shape, deterministic=True)
+    _, _, want = ops.bsa_fwd_tile_stats(qd, kd, vd, full, case.tile_shape, deterministic=True)
+    torch.cuda.synchronize()
+    expected, _ = _oracle_stats(case, q, k, v)
+    _compare_stats(got, expected)
+    torch.testing.assert_close(got["mass"], want["mass"], atol=STAT_ATOL, rtol=2e-3)
+
+
 @pytest.mark.parametrize("grid,tile,deterministic", [
     ((2, 18, 32), 64, True),    # 9 x 8 = 72 tokens: gathered stream
     ((2, 18, 32), 64, False),   # the same with the aligned walk
