@@ -430,8 +430,10 @@ int launch_f32_typed(const BsaParams& p, hipStream_t stream, const char* who) {
 
 }  // namespace bsa
 
-// fp32-compute launches: every call of fp32 inputs (dtype DSA_F32), dense
-// calls with dropout, and calls of head dims 136..256 of any input type.
+// fp32-compute launches: dense calls with dropout and calls of head dims 136..256,
+// of any input type; of fp32 inputs (dtype DSA_F32) also those without the
+// workspace or the size for the split products, and the heads that
+// bsa_fwd_split_kernel leaves.
 int bsa_launch_f32(bsa::BsaParams p, int32_t dtype, hipStream_t stream, const char* who) {
   if (dtype == DSA_F32) return bsa::launch_f32_typed<float>(p, stream, who);
   if (dtype == DSA_F16) return bsa::launch_f32_typed<_Float16>(p, stream, who);

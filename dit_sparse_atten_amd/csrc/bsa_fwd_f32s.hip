@@ -38,8 +38,9 @@
 // 16-bit kernel's 64-key half-tile (bsa_kernel.h): buffer -> LDS loads one
 // sub-tile ahead, K chunks XOR-swizzled, V^T through the transposing read.
 // Measured against the fp32 kernel, same box: dense 14,400 tokens x 12 heads
-// 11.63 -> 3.58 ms (357 TFLOP/s), 3,600 tokens 1.04 -> 0.34 ms; 12,288 tokens
-// in 8 x 8 tiles with statistics 11.9 -> 2.6 ms.
+// 11.59 -> 3.35 ms (380 TFLOP/s), 3,600 tokens 1.00 -> 0.28 ms; 12,288 tokens in
+// 8 x 8 tiles with statistics, routed (keep 0.625) 10.2 -> 2.1 ms, dense 16.2 ->
+// 3.0 ms.
 #include "bsa_kernel.h"
 #include "bsa_split.h"
 
@@ -559,8 +560,11 @@ int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, size_t workspace_byt
   const int slots = device_slots(stream);
   const bool two = p.block <= 64, single = grid > slots;
   // Split last round: a 4-wave workgroup alone on a CU runs nearly twice as fast
-  // as one of two, so a round is one per CU (2-wave ones: two).  3,600 tokens x
-  // 12 heads (348 workgroups, 92 in five parts) 288 -> 242 us.
+  // as one of two, so a round is one per CU (2-wave ones: two).  Whole calls,
+  // dense, us without and with it: 144 workgroups (1,536 tokens x 12 heads) 93 ->
+  // 81, 160 (4,096 x 5) 204 -> 157, 192 (8,192 x 3) 405 -> 317, 192 of 16 key
+  // blocks 121 -> 119, 348 (3,600 x 12) 299 -> 270, 564 (6,000 x 12) 782 -> 628;
+  // 400 of 10 key blocks, 456 and 480 are not split.
   const size_t lead = split_workspace_bytes(pairs, p.kv_tokens);
   p.part = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + lead);
   p.parts = 1;

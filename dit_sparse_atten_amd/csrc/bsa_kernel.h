@@ -37,8 +37,9 @@
 //    the final row sum pair lanes l and l ^ 32 with v_permlane32_swap;
 //  * query / key blocks of 1..128 tokens (the matrix-sparse backend's spatial
 //    tiles): routed whole blocks of 65..127 keys stream the row's kept blocks
-//    as one gathered key sequence (up to 96 in bsa_narrow.h, above kGather), and routed blocks of at most 64
-//    tokens run 2-wave workgroups (kWaves);
+//    as one gathered key sequence (kGather; up to 96 keys, in calls that fill
+//    the chip, bsa_narrow.h), and routed blocks of at most 64 tokens run 2-wave
+//    workgroups (kWaves);
 //  * the last, partial round of query blocks may run as 2..8 key ranges each
 //    (choose_split), whose fp32 partials bsa_merge_kernel combines;
 //  * routed calls may walk each row's key blocks from a rotated start (the
@@ -1332,7 +1333,12 @@ int launch_typed(BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t s
   // fewer, three waves to a tile finish it sooner (72-token tiles, the 32-row
   // gathered stream against bsa_narrow.h: 768 tiles with statistics 238 / 256 us,
   // 192 tiles 86 / 95; 1,056 tiles 384 / 363, 1,200 tiles 457 / 423, 8,000 tiles
-  // 4.78 / 4.30 ms).  The gathered stream also takes blocks of 97..127.
+  // 4.78 / 4.30 ms).  Larger tiles gain less, and still at 96 rows, which fill
+  // three waves (routed, keep 0.65, attention / with statistics; 6,000 tiles in 40
+  // heads, ms): 81 tokens 2.96 -> 2.70 / 3.68 -> 3.39, 88 2.79 -> 2.61 / 3.48 ->
+  // 3.28, 90 3.32 -> 2.91 / 3.93 -> 3.70, 96 3.31 -> 2.85 / 3.88 -> 3.59; 1,800
+  // tiles in 12 heads 81 to 91 tokens 1 to 6% / equal within 2%.  The gathered
+  // stream also takes blocks of 97..127.
   const bool tiles = p.row_ptr || (p.rs_logm && p.stat_tile == p.block);
   const bool narrow = tiles && grid > 2 * device_slots(stream) &&
                       use_narrow(p.block, p.kv_tokens, p.k_st, p.v_st);
@@ -1428,11 +1434,12 @@ int launch_typed(BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t s
 // fp16 instances (bsa_fwd_f16.hip).
 int bsa_launch_f16(bsa::BsaParams p, void* scratch, size_t scratch_bytes, hipStream_t stream,
                    const char* who);
-// fp32-compute kernel (bsa_fwd_f32.hip): fp32 inputs (dtype DSA_F32), dense
-// calls with dropout, and head dims 136..256, of any input type.
+// fp32-compute kernel (bsa_fwd_f32.hip): dense calls with dropout and head dims
+// 136..256, of any input type, and the fp32 calls and heads (dtype DSA_F32) that
+// the split products leave.
 int bsa_launch_f32(bsa::BsaParams p, int32_t dtype, hipStream_t stream, const char* who);
 // Split fp16 products (bsa_fwd_f32s.hip): fp32 inputs, head dims up to 128, no
-// dropout, on at least split_workspace_bytes of workspace.
+// dropout, split_takes, on at least split_workspace_bytes of workspace.
 int bsa_launch_f32_split(bsa::BsaParams p, void* workspace, size_t workspace_bytes,
                          hipStream_t stream, const char* who);
 namespace bsa {

@@ -102,10 +102,10 @@ __device__ __forceinline__ void round_pair(float a, float b, float& ra, float& r
 // block to p.part and, after the scan, reads them back and adds the rows of
 // each query block over their row totals.  Writing and reading 4 bytes per
 // (row, key block) costs far less than the second sweep's rounding, fma, exp
-// and add per score: 57,600 tokens x 40 heads, 16 samples, same
-// box: 1.02 against 1.73 ms.  Without a workspace (kOnce = false; also SP >= 64, whose blocks
-// span waves) sweep 1 builds each query's log-sum-exp and sweep 2 sums the
-// normalised probabilities per (query block, key block).  Three waves per SIMD
+// and add per score: 57,600 tokens x 40 heads, 16 samples, same box: 1.04 against
+// 1.58 ms.  Without a workspace (kOnce = false; also SP >= 64, whose blocks span
+// waves) sweep 1 builds each query's log-sum-exp and sweep 2 sums the normalised
+// probabilities per (query block, key block).  Three waves per SIMD
 // (168 VGPRs): with four, the longer instances spill.
 //
 // kHalves: head dims up to 128 * kHalves.  Head dims above 128 stage each

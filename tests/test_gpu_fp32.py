@@ -1,11 +1,12 @@
-"""GPU parity of the float32 calls (the fp32 matrix-core kernel,
-csrc/bsa_fwd_f32.hip) against float64 closed forms and the oracle.
+"""GPU parity of the float32 calls (split fp16 products, csrc/bsa_fwd_f32s.hip,
+and the fp32 matrix-core kernel, csrc/bsa_fwd_f32.hip) against float64 closed
+forms and the oracle.
 
 The reference computes in the dtype it is given: DenseBackend hands
 ``dtype`` to SDPA (attention_backends/dense.py:34-47) and MatrixSparseBackend
 computes in q's own dtype (sparse.py:700-708), which is how its float32
-golden fixtures were written.  The kernel forms fp32 products with fp32
-accumulation and keeps the probabilities in fp32, so the bar is fp32
+golden fixtures were written.  Either path accumulates in fp32 and holds its
+operands and probabilities to an fp32 rounding or two, so the bar is fp32
 rounding: outputs within 2e-5 of the float64 closed form (values of order
 one), LSE within 2e-5, statistics within rtol 1e-5.
 """
