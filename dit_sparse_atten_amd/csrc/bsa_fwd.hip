@@ -340,7 +340,7 @@ extern "C" size_t dsa_bsa_f32_workspace_bytes_block(int32_t batch, int32_t heads
                                                     int32_t kv_tokens, int32_t head_dim,
                                                     int32_t block_size) {
   if (batch <= 0 || heads <= 0 || kv_tokens <= kSplitFewKeys || head_dim <= 0 ||
-      head_dim > kHeadDim)
+      head_dim > kHeadDim || (head_dim < 64 && kv_tokens < 256))
     return 0;
   if (block_size <= 0 || block_size > 128) return 0;
   const int32_t kv_blocks = (kv_tokens + block_size - 1) / block_size;

@@ -83,18 +83,19 @@ def _workspace(device, size, *less):
     return workspace, workspace.data_ptr(), size
 
 
-def _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim, block_size):
+def _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim, block_size, every_key):
     """Workspace of the float32 attention's split products (0 for the 16-bit
-    types and for head dims above 128)."""
-    if q.dtype != torch.float32:
+    types, for few keys, for head dims above 128, and below 64 unless every row
+    attends every key)."""
+    if q.dtype != torch.float32 or (head_dim < 64 and not every_key):
         return 0
     return lib.dsa_bsa_f32_workspace_bytes_block(batch, heads, kv_tokens, head_dim, block_size)
 
 
-def _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, block_size):
+def _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, block_size, dense):
     """Workspace of an attention call with statistics: ``own`` bytes, in which
     the float32 split products take the place of the 16-bit kernels' scratch."""
-    more = _f32_workspace_bytes(lib, q, 1, heads, tokens, head_dim, block_size)
+    more = _f32_workspace_bytes(lib, q, 1, heads, tokens, head_dim, block_size, dense)
     if more:
         own += max(0, more - lib.dsa_bsa_workspace_bytes_block(1, heads, tokens, head_dim,
                                                                block_size))
@@ -252,7 +253,8 @@ def bsa_fwd(q, k, v, csr=None, scale=None, out=None, return_lse=False, block_siz
     if q.dtype == torch.float32 or head_dim > HEAD_DIM:
         workspace, workspace_ptr, workspace_bytes = _workspace(
             q.device,
-            _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim, block_size), 0)
+            _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim, block_size,
+                                 csr is None and not causal), 0)
     else:
         workspace, workspace_ptr, workspace_bytes = _workspace(
             q.device, lib.dsa_bsa_workspace_bytes_block(batch, heads, kv_tokens, head_dim,
@@ -391,7 +393,7 @@ def bsa_fwd_block_mass(q, k, v, scale=None):
     # the attention and then the block-mass pass.
     own = lib.dsa_bsa_fwd_block_mass_workspace_bytes(heads, tokens, head_dim)
     workspace, workspace_ptr, workspace_bytes = _workspace(
-        q.device, _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, 128),
+        q.device, _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, 128, True),
         own if tokens % 128 == 0 else lib.dsa_bsa_workspace_bytes(1, heads, tokens, head_dim))
     with torch.cuda.device(q.device):
         status = lib.dsa_bsa_fwd_block_mass(
@@ -522,7 +524,8 @@ def bsa_fwd_tile_stats(q, k, v, csr, tile_shape, scale=None, deterministic=False
     own = lib.dsa_bsa_fwd_tile_stats_workspace_bytes(heads, tokens, head_dim, tile_h, tile_w,
                                                      entries)
     workspace, workspace_ptr, workspace_bytes = _workspace(
-        q.device, _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, tile), own)
+        q.device,
+        _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, tile, csr is None), own)
     with torch.cuda.device(q.device):
         status = lib.dsa_bsa_fwd_tile_stats(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),

@@ -141,9 +141,9 @@ size_t dsa_bsa_workspace_bytes_block(int32_t batch, int32_t heads, int32_t kv_to
  * The split K and V take 1,024 bytes per token, batch item and head, and 1,280
  * per batch item and head (rounded up to 256), then 68,157,440 for a split
  * last round (optional) when the key range holds at least 8 blocks (two parts
- * of at least 4 key blocks).  0 above head dim 128 and up to 64 keys, where one
- * launch of the fp32 kernel is the faster (up to 96 keys it also runs calls of at
- * most 256 query blocks).  With less workspace
+ * of at least 4 key blocks).  0 above head dim 128, below 64 with fewer than 256
+ * keys, and up to 64 keys, where one launch of the fp32 kernel is the faster (up
+ * to 96 keys it also runs calls of at most 256 query blocks).  With less workspace
  * (always more than dsa_bsa_workspace_bytes_block() bytes) the fp32 kernel
  * runs, so the workspace a caller gives is the choice between the two.  _block: for any block_size in 1..128. */
 size_t dsa_bsa_f32_workspace_bytes(int32_t batch, int32_t heads, int32_t kv_tokens,

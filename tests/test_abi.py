@@ -78,6 +78,8 @@ def test_f32_workspace_size(lib):
     assert lib.dsa_bsa_f32_workspace_bytes_block(1, 3, 504, 128, 72) == planes(3, 504)
     assert lib.dsa_bsa_f32_workspace_bytes(1, 12, 512, 136) == 0
     assert lib.dsa_bsa_f32_workspace_bytes(1, 12, 64, 128) == 0
+    assert lib.dsa_bsa_f32_workspace_bytes(1, 12, 255, 56) == 0
+    assert lib.dsa_bsa_f32_workspace_bytes(1, 12, 256, 56) == planes(12, 256)
     assert lib.dsa_bsa_f32_workspace_bytes(1, 12, 65, 128) == planes(12, 65)
     # Always more than the 16-bit kernels' workspace, which a float32 call may
     # be given without asking for the split products.

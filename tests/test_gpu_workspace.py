@@ -49,6 +49,21 @@ def test_float32_attention_without_room_for_the_split(ops, cuda_device, monkeypa
     assert torch.equal(got, ops.bsa_fwd(q, k, v))
 
 
+def test_no_float32_workspace_where_the_split_is_not_taken(ops, cuda_device, short_of_memory):
+    """Head dims below 64 with a route or a causal mask, and few keys."""
+    generator = torch.Generator(device=cuda_device).manual_seed(0)
+    q, k, v = (torch.randn(1, 512, 2, 32, device=cuda_device, generator=generator)
+               for _ in range(3))
+    csr = ops.route_to_csr(torch.ones(2, 4, 4, dtype=torch.bool, device=cuda_device))
+    asked = short_of_memory(1 << 40)
+    ops.bsa_fwd(q, k, v, csr)
+    ops.bsa_fwd(q, k, v, causal=True)
+    ops.bsa_fwd(q, k[:, :64], v[:, :64])
+    assert not asked
+    ops.bsa_fwd(q, k, v)
+    assert len(asked) == 1
+
+
 def test_sampled_mass_without_room_for_its_sums(ops, cuda_device, monkeypatch, short_of_memory):
     q, k, _ = _qkv(13312, 40, cuda_device, torch.bfloat16)
     want = ops.sampled_block_mass(q, k, 128, 32)
