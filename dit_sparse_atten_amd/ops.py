@@ -68,19 +68,15 @@ def _kernel_view(name, tensor, dtype=None, attention=False):
     return tensor if ok else tensor.contiguous()
 
 
-def _workspace(device, size, *less):
-    """(workspace, its data pointer, its bytes): ``size`` bytes, or the first of
-    ``less`` that the device has memory for, where a call has another way with
-    them (0: none; without ``less`` it has not)."""
-    if not size:
-        return None, None, 0
-    try:
-        workspace = torch.empty(size, dtype=torch.uint8, device=device)
-    except torch.OutOfMemoryError:
-        if not less:
-            raise
-        return _workspace(device, *less)
-    return workspace, workspace.data_ptr(), size
+def _smaller_workspace(device, *sizes):
+    """A workspace of the first of ``sizes`` (descending; 0: None) that the device
+    has memory for, of a call that has another way with it."""
+    for index, size in enumerate(sizes):
+        try:
+            return torch.empty(size, dtype=torch.uint8, device=device) if size else None
+        except torch.OutOfMemoryError:
+            if index + 1 == len(sizes):
+                raise
 
 
 def _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim, block_size, every_key):
@@ -250,15 +246,20 @@ def bsa_fwd(q, k, v, csr=None, scale=None, out=None, return_lse=False, block_siz
     # the key range is too short to split), or, in fp32, for the split K and V
     # (head dims above 128 run the fp32-compute kernel, which uses none); the
     # caching allocator recycles it.
-    if q.dtype == torch.float32 or head_dim > HEAD_DIM:
-        workspace, workspace_ptr, workspace_bytes = _workspace(
-            q.device,
-            _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim, block_size,
-                                 csr is None and not causal), 0)
+    fp32_kernel = q.dtype == torch.float32 or head_dim > HEAD_DIM
+    if fp32_kernel:
+        workspace_bytes = _f32_workspace_bytes(lib, q, batch, heads, kv_tokens, head_dim,
+                                               block_size, csr is None and not causal)
     else:
-        workspace, workspace_ptr, workspace_bytes = _workspace(
-            q.device, lib.dsa_bsa_workspace_bytes_block(batch, heads, kv_tokens, head_dim,
-                                                        block_size))
+        workspace_bytes = lib.dsa_bsa_workspace_bytes_block(
+            batch, heads, kv_tokens, head_dim, block_size)
+    try:
+        workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device)
+                     if workspace_bytes else None)
+    except torch.OutOfMemoryError:
+        if not fp32_kernel:
+            raise
+        workspace, workspace_bytes = None, 0  # float32 products
     with torch.cuda.device(q.device):
         status = lib.dsa_bsa_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
@@ -267,7 +268,8 @@ def bsa_fwd(q, k, v, csr=None, scale=None, out=None, return_lse=False, block_siz
             row_ptr.data_ptr() if row_ptr is not None else None,
             col_idx.data_ptr() if col_idx is not None else None,
             route_batches, float(scale), int(bool(causal)), int(bool(deterministic)),
-            lse.data_ptr() if lse is not None else None, workspace_ptr, workspace_bytes,
+            lse.data_ptr() if lse is not None else None,
+            workspace.data_ptr() if workspace is not None else None, workspace_bytes,
             _stream_handle(q.device))
     _lib.check(status, "dsa_bsa_fwd")
     return (out, lse) if return_lse else out
@@ -307,12 +309,18 @@ def sampled_block_mass(q, k, block_size, samples=2, scale=None):
     strides = _lib.int64_array([q.stride(1), q.stride(2), k.stride(1), k.stride(2)])
     # Row sums of a single scan (none above 32 samples, which scan twice): with
     # half in several launches, without any in two scans.
-    full = _sampled_mass_workspace_bytes(tokens, heads, block_size, samples)
-    workspace, workspace_ptr, workspace_bytes = _workspace(q.device, full, full // 2, 0)
+    workspace_bytes = _sampled_mass_workspace_bytes(tokens, heads, block_size, samples)
+    try:
+        workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device)
+                     if workspace_bytes else None)
+    except torch.OutOfMemoryError:
+        workspace = _smaller_workspace(q.device, workspace_bytes // 2, 0)
+        workspace_bytes = workspace.numel() if workspace is not None else 0
     with torch.cuda.device(q.device):
         status = lib.dsa_sampled_mass_ws(
             q.data_ptr(), k.data_ptr(), dtype_code(q.dtype), strides, tokens, heads, head_dim, block_size,
-            samples, float(scale), mass.data_ptr(), workspace_ptr, workspace_bytes,
+            samples, float(scale), mass.data_ptr(),
+            workspace.data_ptr() if workspace is not None else None, workspace_bytes,
             _stream_handle(q.device))
     _lib.check(status, "dsa_sampled_mass")
     return mass
@@ -389,18 +397,24 @@ def bsa_fwd_block_mass(q, k, v, scale=None):
     strides = _lib.int64_array(
         list(q.stride()[:3]) + list(k.stride()[:3]) + list(v.stride()[:3])
         + list(out.stride()[:3]))
-    # With less than its own bytes: float32 products, or (a partial last block)
-    # the attention and then the block-mass pass.
-    own = lib.dsa_bsa_fwd_block_mass_workspace_bytes(heads, tokens, head_dim)
-    workspace, workspace_ptr, workspace_bytes = _workspace(
-        q.device, _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, 128, True),
-        own if tokens % 128 == 0 else lib.dsa_bsa_workspace_bytes(1, heads, tokens, head_dim))
+    workspace_bytes = own = lib.dsa_bsa_fwd_block_mass_workspace_bytes(heads, tokens, head_dim)
+    if q.dtype == torch.float32:
+        workspace_bytes = _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, 128,
+                                                      True)
+    try:
+        workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device)
+    except torch.OutOfMemoryError:
+        # float32 products; a partial last block: the attention, then a second pass.
+        workspace = _smaller_workspace(
+            q.device,
+            own if tokens % 128 == 0 else lib.dsa_bsa_workspace_bytes(1, heads, tokens, head_dim))
+        workspace_bytes = workspace.numel()
     with torch.cuda.device(q.device):
         status = lib.dsa_bsa_fwd_block_mass(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
             dtype_code(q.dtype, attention=True),
             strides, tokens, heads, head_dim, float(scale), lse.data_ptr(), mass.data_ptr(),
-            workspace_ptr, workspace_bytes, _stream_handle(q.device))
+            workspace.data_ptr(), workspace_bytes, _stream_handle(q.device))
     _lib.check(status, "dsa_bsa_fwd_block_mass")
     return out, lse, mass
 
@@ -521,11 +535,18 @@ def bsa_fwd_tile_stats(q, k, v, csr, tile_shape, scale=None, deterministic=False
     strides = _lib.int64_array(
         list(q.stride()[:3]) + list(k.stride()[:3]) + list(v.stride()[:3])
         + list(out.stride()[:3]))
-    own = lib.dsa_bsa_fwd_tile_stats_workspace_bytes(heads, tokens, head_dim, tile_h, tile_w,
-                                                     entries)
-    workspace, workspace_ptr, workspace_bytes = _workspace(
-        q.device,
-        _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, tile, csr is None), own)
+    workspace_bytes = own = lib.dsa_bsa_fwd_tile_stats_workspace_bytes(
+        heads, tokens, head_dim, tile_h, tile_w, entries)
+    if q.dtype == torch.float32:
+        workspace_bytes = _statistics_workspace_bytes(lib, q, own, heads, tokens, head_dim, tile,
+                                                      csr is None)
+    try:
+        workspace = (torch.empty(workspace_bytes, dtype=torch.uint8, device=q.device)
+                     if workspace_bytes else None)
+    except torch.OutOfMemoryError:
+        if workspace_bytes == own:
+            raise
+        workspace, workspace_bytes = _smaller_workspace(q.device, own), own  # float32 products
     with torch.cuda.device(q.device):
         status = lib.dsa_bsa_fwd_tile_stats(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
@@ -535,7 +556,8 @@ def bsa_fwd_tile_stats(q, k, v, csr, tile_shape, scale=None, deterministic=False
             entries, float(scale), int(bool(deterministic)),
             lse.data_ptr(), stats["mass"].data_ptr(), stats["mass_f16"].data_ptr(),
             *[stats[name].data_ptr() if name in stats else None for name in names],
-            workspace_ptr, workspace_bytes, _stream_handle(q.device))
+            workspace.data_ptr() if workspace is not None else None, workspace_bytes,
+            _stream_handle(q.device))
     _lib.check(status, "dsa_bsa_fwd_tile_stats")
     return out, lse, stats
 
