@@ -103,8 +103,8 @@ __device__ __forceinline__ void round_pair(float a, float b, float& ra, float& r
 // block to p.part and, after the scan, reads them back and adds the rows of
 // each query block over their row totals.  Writing and reading 4 bytes per
 // (row, key block) costs far less than the second sweep's rounding, fma, exp
-// and add per score: 57,600 tokens x 40 heads, 16 samples, same box: 1.04 against
-// 1.58 ms.  Without a workspace (kOnce = false; also SP >= 64, whose blocks span
+// and add per score: 57,600 tokens x 40 heads, 16 samples: 1.04 ms (0.8 with the
+// fences below at workgroup scope) against 1.58 ms.  Without a workspace (kOnce = false; also SP >= 64, whose blocks span
 // waves) sweep 1 builds each query's log-sum-exp and sweep 2 sums the normalised
 // probabilities per (query block, key block).  Three waves per SIMD
 // (168 VGPRs): with four, the longer instances spill.
@@ -218,10 +218,13 @@ __global__ void __launch_bounds__(256, kHalves == 1 ? 3 : 2) sampled_mass_kernel
   // kOnce: this wave's row sums [key block][32 rows].
   float* const part =
       kOnce ? p.part + ((int64_t)blockIdx.x * 4 + wave) * 32 * part_blocks(p.blocks) : nullptr;
-  // Makes the wave's own stores to `part` visible to its loads.
+  // Makes the wave's own stores to `part` visible to its other lanes' loads.  At
+  // workgroup scope, as one L1 serves them: at agent scope every wave wrote back
+  // and invalidated its XCD's L2, beside the kernels of other streams (a whole
+  // route update at 57,600 tokens x 40 heads 1,179 us, with this 957).
   auto settle_part = [&]() __attribute__((always_inline)) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   };
 
   // One tile; kTail: it may hold keys of the last block, padding slots or
